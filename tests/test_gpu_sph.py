@@ -306,6 +306,72 @@ def test_prefilter_keeps_pairs_at_the_cut_exact():
             assert np.array_equal(s.get("objectPointing"), want), (pre, L)
 
 
+@pytest.mark.parametrize("two_h", [False, True])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 7, 8, 9, 31, 33, 65, 300, 6001])
+def test_lists_at_slot_edges_and_outside_the_grid(n, two_h):
+    """Particle counts about the list build's wave widths (4, 8, 16, 32 and 64
+    slots; 6,001 is past its four-slot rule) with one particle in five outside
+    the grid: a fraction of a cell to 20 cells off, on both sides of the 10.5
+    and 12 cells at which a point stops taking plain tests, in tight pairs
+    there, and on the maximum faces.  Whole numbers: lists equal the oracle's
+    at every lane count, one and two smoothing lengths."""
+    rng = np.random.default_rng(1000 + n)
+    dx = 0.01
+    cell = 2.0 * 1.3 * dx
+    side = max(3.2 * cell, 0.75 * dx * n ** (1.0 / 3.0))
+    pos = rng.uniform(0.0, side, (n, 3))
+    off = np.flatnonzero(rng.random(n) < 0.2)
+    ax = rng.integers(0, 3, len(off))
+    d = cell * rng.choice([0.3, 1.2, 2.0, 4.0, 10.45, 10.55, 11.9, 12.1, 20.0], len(off)) * rng.uniform(0.97, 1.03, len(off))
+    up = rng.random(len(off)) < 0.5
+    pos[off, ax] = np.where(up, side + d, -d)
+    pos[off[1::2]] = pos[off[:len(off) // 2 * 2:2]] + rng.uniform(-0.4, 0.4, (len(off) // 2, 3)) * cell
+    if n > 8:
+        pos[off[0], :2] = side
+    g = np.arange(0.0, side, dx)
+    dummy = np.stack(np.meshgrid(g, g, [0.5 * dx], indexing="ij"), -1).reshape(-1, 3)
+    spec = scenes.SPHSceneSpec(fluid_pos=pos, dummy_pos=dummy, dx=dx, rho0=1000.0, c0=10.0, nu=1e-6, min_bound=np.zeros(3),
+                               max_bound=np.full(3, side), gravity=np.array([0.0, 0.0, -9.81]), dt=1e-5)
+    if two_h:
+        w = rng.random(n) < 0.5
+        spec.fluid_dx = np.where(w, dx, 0.8 * dx)
+        spec.fluid_rho0 = np.where(w, 1000.0, 900.0)
+    o = oracle.OracleSPH(spec)
+    o.neighbor_search()
+    for L in (0, 1, 2, 4, 8):
+        s = make_gpu(spec)
+        s.tune("listLanes", L)
+        s.neighbor_search()
+        assert np.array_equal(s.get("neighborCount"), o.get("count_ff")), L
+        assert np.array_equal(s.get("objectPointing"), o.get("pointing_ff")), L
+        assert np.array_equal(s.get("dummyNeighborCount"), o.get("count_fd")), L
+        assert np.array_equal(s.get("dummyObjectPointing"), o.get("pointing_fd")), L
+
+
+@pytest.mark.parametrize("field", ["velocity", "densityChange"])
+def test_records_follow_a_field_set_between_search_and_halves(field, small):
+    """A field set after the search reaches the records that the passes
+    gather.  The two forms of the pair passes differ by the rounding of FP32
+    sums over about 80 pairs, 80 x 6e-8 of the largest term: 1e-5 of the
+    largest value bounds it, and a stale field would miss by its change."""
+    rng = np.random.default_rng(9)
+    got = []
+    value = None
+    for rec in (1, 0):
+        s = make_gpu(small)
+        s.tune("pairRecords", rec)
+        s.neighbor_search()
+        if value is None:
+            old = s.get(field)
+            value = old + rng.uniform(-0.5, 0.5, old.shape)
+        s.set(field, value)
+        s.first_half(small.dt)
+        s.second_half(small.dt)
+        got.append([s.get(f) for f in ("velocity", "density")])
+    for a, b in zip(*got):
+        assert np.abs(a - b).max() < 1e-5 * np.abs(b).max()
+
+
 def test_two_phases_match_oracle():
     """Two fluid phases of different spacing, density and viscosity side by
     side (the kernels' non-uniform paths: per-pair cuts, phase lookups,

@@ -258,6 +258,18 @@ __device__ __forceinline__ int xcd_block()
     return (xcd < r) ? xcd * (q + 1) + pos : r * (q + 1) + (xcd - r) * q + pos;
 }
 
+// The same with each XCD's share spread over the whole range in runs of RUN
+// consecutive logical blocks, for work that is uneven along the range.
+template <int RUN>
+__device__ __forceinline__ int xcd_block_spread()
+{
+    const int b = blockIdx.x, G = gridDim.x;
+    const int whole = G / (kNumXcd * RUN) * (kNumXcd * RUN);
+    if (b >= whole) return b;
+    const int xcd = b % kNumXcd, pos = b / kNumXcd;
+    return (pos / RUN * kNumXcd + xcd) * RUN + pos % RUN;
+}
+
 inline int blocks_for(long long n, int threads) { return (int)((n + threads - 1) / threads); }
 
 // ---------------------------------------------------------------- sort/scan

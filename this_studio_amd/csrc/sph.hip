@@ -16,13 +16,14 @@
 //   drho      f32[n]                         own-slot only
 // Dummies (sorted once): DummyPos {x, y, z: f64; nx, ny: f32} and float4
 // {vx, vy, vz, nz}.
-// Neighbour lists are ELL in 32-byte chunks: entries 8c..8c+7 of slot i sit
-// at int offset (c*n + i)*8.  The list kernel fills a chunk in registers and
-// stores it whole, so every store covers full 32-byte sectors; the lanes of
-// a wavefront read one chunk of consecutive slots as consecutive 16-byte
-// words.  Each slot's list holds neighbour slots in the reference's exact
-// walk order (z, y, x cells, then ascending insertion index), so the pair
-// set and its per-particle order are identical to the reference's.
+// Neighbour lists hold K entries per slot in 32-byte chunks of eight, those
+// of 16 consecutive slots interleaved (list_entry): the lanes of a wavefront
+// read one chunk of consecutive slots as consecutive 16-byte words, and the
+// list build finds an entry with one multiply-add.  Each slot's list holds neighbour slots in the reference's
+// exact walk order (z, y, x cells, then ascending insertion index), so the
+// pair set and its per-particle order are identical to the reference's.  The
+// lists of coupled balls are ELL in 32-byte chunks: entries 8c..8c+7 of slot
+// i at int offset (c*n + i)*8.
 //
 // Pair arithmetic is FP32 (positions differenced in FP64 first); state
 // integration is FP64.
@@ -82,35 +83,105 @@ struct alignas(32) SolidPos {
 };
 static_assert(sizeof(SolidPos) == 32, "SolidPos is one 32-byte record");
 
-// The 32-byte record a pair pass gathers for a fluid neighbour (uniform
-// scenes): the position as an FP32 offset from the origin of the particle's
-// cell at the last sort, density, pressure and velocity.  Two 16-byte loads
+// Fixed-point positions.  A coordinate is stored as the low 32 bits of
+// round((x - min) / u), with 2^25 to 2^26 units u to the largest cell edge:
+// positions modulo 64 cells or more, at most 3e-8 cells (8e-8 spacings) apart.  Everything that compares two
+// positions meets them within one 27-cell stencil, where the wrapped 32-bit
+// difference is the true one, exact to one unit however large the grid: an
+// integer subtraction and a conversion where offsets from cell origins took
+// the neighbour's cell out of the list entry and nine FP32 operations.
+//
+// A point is "far" when that argument does not cover it: more than 10.5 cells
+// outside the grid on some axis (its hash is clamped into the face cells; 12
+// cells on both sides plus a stencil stay far below the 64-cell period), on
+// the rounding edge of the maximum face (where the hash can land in another
+// row of cells), or not a number.  Far points take the FP64 test in the list
+// build, and a particle that is far or lists a far neighbour takes the FP64
+// records in the pair passes (kFarBit of its count).  Beyond 12 cells, or not
+// a number, it is "out": farther than any cut from every point that is not far.
+constexpr double kFixPerCell = 67108864.0;  // 2^26: units to a cell edge, at most
+constexpr double kFixPad = 12.0 * kFixPerCell, kFixNear = 10.5 * kFixPerCell;
+struct FixGeom {
+    double minx, miny, minz;
+    double ex, ey, ez;  // extent of the grid in units
+    double inv;         // units per metre
+    float u;            // metres per unit
+};
+struct Fix3 {
+    int x, y, z;
+    bool far, out;
+};
+__device__ __forceinline__ int fix_coord(double X)
+{
+    const double y = X + 0.5;
+    return (int)(unsigned)(y - 4294967296.0 * floor(y * (1.0 / 4294967296.0)));
+}
+__device__ __forceinline__ bool fix_out(double X, double E) { return !(X >= -kFixPad && X <= E + kFixPad); }
+__device__ __forceinline__ bool fix_edge(double X, double E)
+{
+    return fabs(X - E) < 4.0 || X < -kFixNear || X > E + kFixNear;
+}
+__device__ __forceinline__ Fix3 fix_pos(const FixGeom& f, double x, double y, double z)
+{
+    const double X = (x - f.minx) * f.inv, Y = (y - f.miny) * f.inv, Z = (z - f.minz) * f.inv;
+    const bool out = fix_out(X, f.ex) || fix_out(Y, f.ey) || fix_out(Z, f.ez);
+    return Fix3{fix_coord(X), fix_coord(Y), fix_coord(Z),
+                out || fix_edge(X, f.ex) || fix_edge(Y, f.ey) || fix_edge(Z, f.ez), out};
+}
+
+// The 32-byte record of a fluid particle: fixed-point position and density,
+// pressure and velocity.  The list build reads the first half of every
+// scene; the pair passes of uniform scenes gather both, two 16-byte loads
 // per neighbour where the FP64 position, density and pressure (32 bytes)
-// plus the velocity (12) take three; the pair passes issue about one
-// vector-L1 line access per CU per cycle, so the loads per neighbour set
-// their time.  A list entry then carries the neighbour's cell relative to
-// the particle's stencil centre, 2 bits per axis above the slot, and
-// x_i - x_j = (o_i - o_j) - (c_j - c_i) cs: the offsets are below 2 cells,
-// so the difference keeps ~1e-9 m absolute (3e-7 of a typical pair
-// distance), against 3e-8 relative when rounding the FP64 difference.
+// plus the velocity (12) take three.
 //
 // The two 16-byte halves of the records lie in two arrays of nf float4 (one
-// buffer: {ox, oy, oz, rho} at [0, nf), {p, vx, vy, vz} at [nf, 2 nf)): a
+// buffer: {qx, qy, qz, rho} at [0, nf), {p, vx, vy, vz} at [nf, 2 nf)): a
 // lane group's neighbours are mostly consecutive slots, so each gather
-// instruction touches half the cache lines of 32-byte records.
+// instruction touches half the cache lines of 32-byte records.  The record
+// of a far point written by the sort has a density of -1 (so has one whose
+// density is not positive), of one that is out -2 (fix_mark).
 struct alignas(32) GRec {
-    float ox, oy, oz, rho;
+    int qx, qy, qz;
+    float rho;
     float p, vx, vy, vz;
 };
 static_assert(sizeof(GRec) == 32, "GRec is two 16-byte halves");
-__device__ __forceinline__ void st_grec(float4* base, int half, int k, const GRec& r)
+__device__ __forceinline__ float4 fix_half(const Fix3& q, float w)
 {
-    base[k] = make_float4(r.ox, r.oy, r.oz, r.rho);
-    base[half + k] = make_float4(r.p, r.vx, r.vy, r.vz);
+    return make_float4(__int_as_float(q.x), __int_as_float(q.y), __int_as_float(q.z), w);
 }
-constexpr int kCodeShift = 25;                      // entry = slot | code << 25
-constexpr int kSlotMask = (1 << kCodeShift) - 1;    // slots below 2^25
-__host__ __device__ constexpr int pack_cell(int ix, int iy, int iz) { return ix | iy << 11 | iz << 22; }
+__device__ __forceinline__ float fix_mark(const Fix3& q, float w)
+{
+    return q.out ? -2.0f : q.far || !(w > 0.0f) ? -1.0f : w;
+}
+__device__ __forceinline__ void st_grec(float4* base, int half, int k, const FixGeom& f, const FluidPos& p,
+                                        const float4& v)
+{
+    base[k] = fix_half(fix_pos(f, p.x, p.y, p.z), p.rho);
+    base[half + k] = make_float4(p.p, v.x, v.y, v.z);
+}
+// Entry k of slot i in the neighbour lists of capacity K (a multiple of 8).
+// Rows of K entries instead, each slot's list by itself, made a chunk load of
+// 16 slots touch 16 cache lines that were gone before the next chunk was
+// read: 1.5 times the L2 requests in the momentum passes, twice in the
+// continuity pass.
+constexpr int kListRows = 16;
+constexpr int kListStride = kListRows * kChunk;  // from a chunk to the slot's next
+__host__ __device__ constexpr size_t list_entry(int i, int k, int K)
+{
+    return (size_t)(i / kListRows) * kListRows * K + (size_t)(k / kChunk) * kListStride + i % kListRows * kChunk +
+           k % kChunk;
+}
+// Allocation: whole groups of slots, and one batch of 64 entries beyond a
+// full last list (see the list build).
+constexpr size_t list_alloc(int n, int K)
+{
+    return list_entry((n + kListRows - 1) / kListRows * kListRows, 0, K) + (64 / kChunk + 1) * (size_t)kListStride;
+}
+// Set in a particle's neighbour count when its pairs need the FP64 records.
+constexpr int kFarBit = 1 << 30;
+__host__ __device__ constexpr int list_count(int c) { return c & (kFarBit - 1); }
 
 __device__ __forceinline__ unsigned phase_bits(float w) { return __float_as_uint(w); }
 
@@ -131,15 +202,18 @@ struct SphArgs {
     // lists
     const int *nbr_ff, *cnt_ff, *nbr_fd, *cnt_fd;
     int K_ff, K_fd;
-    // gather records (null: FP64 records): read and written by the passes,
-    // each particle's packed cell at the last sort and stencil centre
+    // gather records (null: FP64 records), read and written by the passes
     const float4* GRin;  // split halves, nf float4 apart
     float4* GRout;
-    const int *pcell, *pcen;
-    GridGeom grid;
+    FixGeom fix;
+    // fluid and dummy pairs on records: u / 2h, u m_j times the kernel constant (GradK)
+    float ff_half_invh, ff_coef, fd_half_invh, fd_coef;
     // dummies (sorted once)
     const DummyPos* DP;
     const float4* DV;
+    // their records: {qx, qy, qz, -}, {nx, ny, nz, vx}, {vy, vz}
+    const float4 *DA, *DB;
+    const float2* DC;
     const uint8_t* dphase;
     // coupled DEM balls (solids), sorted into the fluid grid each step
     int ns;
@@ -168,7 +242,7 @@ __device__ __forceinline__ float rsq(float x) { return __builtin_amdgcn_rsqf(x);
 struct GradK {
     float half_invh, coef, two_h;
 };
-__device__ __forceinline__ GradK grad_k(float h)
+__host__ __device__ inline GradK grad_k(float h)
 {
     GradK k;
     const float invh = 1.0f / h;
@@ -317,34 +391,6 @@ __global__ __launch_bounds__(kThreads) void k_hash(int n, GridGeom g, long long 
     key[orig[s]] = (uint32_t)cell_hash(g, p.x, p.y, p.z);
 }
 
-// FP32 copy of a position relative to the grid origin for the list
-// prefilter; w = 1 marks a point farther than R from the origin on some
-// axis, where the FP32 rounding could reach the prefilter's band.
-__device__ __forceinline__ float4 pos_f32(const GridGeom& g, double R, double x, double y, double z)
-{
-    const double rx = x - g.minx, ry = y - g.miny, rz = z - g.minz;
-    const bool far = fabs(rx) > R || fabs(ry) > R || fabs(rz) > R;
-    return make_float4((float)rx, (float)ry, (float)rz, far ? 1.f : 0.f);
-}
-
-// Origin of a packed cell, and a particle's gather record in it.
-__device__ __forceinline__ void cell_origin(const GridGeom& g, int pc, double& x, double& y, double& z)
-{
-    x = g.minx + (double)(pc & 2047) * g.cx;
-    y = g.miny + (double)((pc >> 11) & 2047) * g.cy;
-    z = g.minz + (double)((pc >> 22) & 1023) * g.cz;
-}
-__device__ __forceinline__ GRec grec(const GridGeom& g, int pc, const FluidPos& p, const float4& v)
-{
-    double x0, y0, z0;
-    cell_origin(g, pc, x0, y0, z0);
-    GRec r;
-    r.ox = (float)(p.x - x0); r.oy = (float)(p.y - y0); r.oz = (float)(p.z - z0);
-    r.rho = p.rho; r.p = p.p;
-    r.vx = v.x; r.vy = v.y; r.vz = v.z;
-    return r;
-}
-
 struct ReorderArgs {
     int n;
     long long numGrids;
@@ -361,11 +407,9 @@ struct ReorderArgs {
     double *ovx, *ovy, *ovz;
     float* odrho;
     int2* cells;  // (start, end) per cell
-    float4* oPf;  // FP32 positions for the list prefilter (null: none)
-    GridGeom grid;
-    double R;
-    float4* oGR;  // gather records (split halves, n apart) and packed cells (null: none)
-    int* opcell;
+    FixGeom fix;
+    float4* oGR;   // records (split halves, n apart)
+    int rec_full;  // the pair passes gather records: write the second half too
 };
 
 __global__ __launch_bounds__(kThreads) void k_reorder(ReorderArgs a)
@@ -378,24 +422,28 @@ __global__ __launch_bounds__(kThreads) void k_reorder(ReorderArgs a)
     a.orig_out[k] = o;
     const FluidPos p = a.P[s];
     a.oP[k] = p;
-    if (a.oPf) a.oPf[k] = pos_f32(a.grid, a.R, p.x, p.y, p.z);
-    a.oV[k] = a.V[s];
+    const float4 v = a.V[s];
+    a.oV[k] = v;
+    const Fix3 q = fix_pos(a.fix, p.x, p.y, p.z);
+    a.oGR[k] = fix_half(q, fix_mark(q, p.rho));
+    if (a.rec_full) a.oGR[a.n + k] = make_float4(p.p, v.x, v.y, v.z);
     a.ovx[k] = a.vx[s]; a.ovy[k] = a.vy[s]; a.ovz[k] = a.vz[s];
     a.odrho[k] = a.drho[s];
     // findStartAndEnd (buildHashStartEnd.cu:14-34)
     const uint32_t h = a.skey[k];
-    if (a.oGR) {
-        const int nxy = a.grid.nx * a.grid.ny;
-        const int hh = (int)h, iz = hh / nxy, r = hh - iz * nxy, iy = r / a.grid.nx, ix = r - iy * a.grid.nx;
-        const int pc = pack_cell(ix, iy, iz);
-        a.opcell[k] = pc;
-        const float4 v = a.V[s];
-        st_grec(a.oGR, a.n, k, grec(a.grid, pc, p, v));
-    }
     if ((long long)h < a.numGrids) {
         if (k == 0 || a.skey[k - 1] != h) a.cells[h].x = k;
         if (k == a.n - 1 || a.skey[k + 1] != h) a.cells[h].y = k + 1;
     }
+}
+
+// Both halves of every record from the current state (after a host write
+// between a search and the passes).
+__global__ __launch_bounds__(kThreads) void k_refresh_records(int n, FixGeom f, const FluidPos* __restrict__ P,
+                                                              const float4* __restrict__ V, float4* GR)
+{
+    const int k = blockIdx.x * kThreads + threadIdx.x;
+    if (k < n) st_grec(GR, n, k, f, P[k], V[k]);
 }
 
 // ----------------------------------------------------------- neighbour lists
@@ -419,15 +467,16 @@ struct ListArgs {
     const SolidPos* SP;
     int *nbr_fs, *cnt_fs;
     int K_fs;
-    // FP32 prefilter of the lane walks: positions relative to the grid
-    // origin (w = 1: far from it), and the relative half-width of the band
-    // around cut^2 in which the exact FP64 test decides
-    const float4 *Pf, *DPf;
-    float band;
-    int* pcen;  // coded lists: each particle's packed stencil centre (null: plain slots)
+    // fixed-point positions (first record halves) of fluid and dummies
+    const float4 *A, *DA;
+    const uint32_t* skey;  // sorted cell hashes
+    long long numGrids;
+    double inv;     // units per metre
+    unsigned long long stepx, stepy, stepz;  // cell edges in 2^-20 units
+    int prefilter;  // 0: every candidate takes the FP64 test
+    float reach, err;  // of a plain test: largest own coordinate, error bound (list_error)
+    float lo_f, hi_f, lo_d, hi_d;  // cut bands of uniform scenes (cut_band)
 };
-
-enum WalkKind { kFluid = 0, kDummy = 1, kSolid = 2 };
 
 // One 32-byte list chunk held in registers while it fills.
 struct Chunk {
@@ -444,49 +493,34 @@ struct Chunk {
     }
 };
 
-// Walks the 27-cell stencil of one point over one sorted set and appends
-// every member within 2*max(hA,hB) to the point's chunked list
-// (SPHNeighborSearchKernel.cu:57-115 with excludeSelf, :169-228 without).
+// Walks the 27-cell stencil of one point over the sorted balls and appends
+// every ball within the fluid's support 2 h to the point's chunked list.
 // The three x-cells of a stencil row are consecutive hashes, so their
 // members form one contiguous run of slots, walked in ascending order: the
 // nine row runs are resolved first (all cell-range loads in flight at
 // once), then each run is walked kWalkAhead candidates at a time with
 // their position loads issued before any test.
-#ifndef DEMSPH_WALK_AHEAD
-#define DEMSPH_WALK_AHEAD 4
-#endif
-constexpr int kWalkAhead = DEMSPH_WALK_AHEAD;
-// Candidates per lane per batch in the lane-group walk.  Three beat four
-// and two (256k points, 4 lanes: 130, 155 and 135 us; 741k: 324, 393 and
-// 332 us): fewer values in flight keep more waves resident and waste less
-// of each row's last batch.
-constexpr int kLaneAhead = 3;
-
-template <bool UNIF, int KIND, class PosT, bool CODED = false>
-__device__ __forceinline__ int walk_list(const ListArgs& a, const PosT* __restrict__ B,
-                                         const int2* __restrict__ cells, double x, double y, double z, double hA,
-                                         int self, int* __restrict__ out, int K)
+constexpr int kWalkAhead = 4;
+__device__ __forceinline__ int walk_solids(const ListArgs& a, double x, double y, double z, double h,
+                                           int* __restrict__ out, int K)
 {
     const GridGeom& g = a.grid;
-    // balls couple to the fluid particles within the fluid's support 2 h_A
-    const double cut_u = KIND == kSolid ? 2.0 * hA : 2.0 * fmax(hA, KIND == kDummy ? a.hd : a.hf);
+    const double cut = 2.0 * h;
     const size_t cstride = (size_t)a.nf * kChunk;
     const int nchunks = K / kChunk;
     const Stencil st = make_stencil(g, x, y, z);
-    int rs[9], re[9], rb0[9], rb1[9];
+    int rs[9], re[9];
 #pragma unroll
     for (int k = 0; k < 9; k++) {
         const int dz = k / 3 - 1, dy = k % 3 - 1;
         const bool row_ok = dz >= st.loz && dz <= st.hiz && dy >= st.loy && dy <= st.hiy;
         const int row = (st.cz + dz) * g.ny * g.nx + (st.cy + dy) * g.nx + st.cx;
         int s = -1, e = -1;
-        int2 rr[3];
 #pragma unroll
         for (int dx = -1; dx <= 1; dx++) {
             const bool ok = row_ok && dx >= st.lox && dx <= st.hix;
-            const int2 c = cells[ok ? row + dx : 0];
+            const int2 c = a.scells[ok ? row + dx : 0];
             const int2 r = ok ? c : make_int2(-1, -1);
-            rr[dx + 1] = r;
             if (r.x != -1) {
                 if (s < 0) s = r.x;
                 e = r.y;
@@ -494,35 +528,26 @@ __device__ __forceinline__ int walk_list(const ListArgs& a, const PosT* __restri
         }
         rs[k] = s < 0 ? 0 : s;
         re[k] = s < 0 ? 0 : e;
-        // a slot's x-cell in the row: -1 below b0, 0 below b1, +1 above
-        rb0[k] = rr[0].x != -1 ? rr[0].y : rs[k];
-        rb1[k] = rr[1].x != -1 ? rr[1].y : rb0[k];
     }
     Chunk buf{0, 0, 0, 0, 0, 0, 0, 0};
     int count = 0;
 #pragma unroll
     for (int k = 0; k < 9; k++) {
         const int e = re[k];
-        const int rowcode = ((k / 3) << 4) | ((k % 3) << 2);  // (dz + 1) << 4 | (dy + 1) << 2
         for (int j0 = rs[k]; j0 < e; j0 += kWalkAhead) {
             double qx[kWalkAhead], qy[kWalkAhead], qz[kWalkAhead];
 #pragma unroll
             for (int u = 0; u < kWalkAhead; u++) {
-                const PosT* b = B + min(j0 + u, e - 1);
+                const SolidPos* b = a.SP + min(j0 + u, e - 1);
                 qx[u] = b->x; qy[u] = b->y; qz[u] = b->z;
             }
 #pragma unroll
             for (int u = 0; u < kWalkAhead; u++) {
                 const int j = j0 + u;
-                if (j >= e || (KIND == kFluid && j == self)) continue;
-                double cut = cut_u;
-                if (!UNIF && KIND != kSolid) {
-                    const double hB = KIND == kDummy ? a.phases[a.dphase[j]].h : a.phases[phase_bits(a.V[j].w)].h;
-                    cut = 2.0 * fmax(hA, hB);
-                }
+                if (j >= e) continue;
                 if (!within_cut(cut, x - qx[u], y - qy[u], z - qz[u])) continue;
                 const int c = count & (kChunk - 1);
-                buf.put(c, CODED ? j | (rowcode | (j >= rb0[k]) + (j >= rb1[k])) << kCodeShift : j);
+                buf.put(c, j);
                 count++;
                 if (c == kChunk - 1) {
                     const int cc = (count >> 3) - 1;
@@ -535,171 +560,357 @@ __device__ __forceinline__ int walk_list(const ListArgs& a, const PosT* __restri
     return count;
 }
 
-// walk_list over L lanes of one point: in each run the lanes test
-// consecutive candidates (kLaneAhead per lane in flight), and a ballot over
-// the lane group ranks the hits, so the list holds the same entries in the
-// same order as walk_list's; entries are stored one int at a time.
-//
-// PRE: candidates are first tested in FP32 on the prefilter copy Bf; only
-// those within the band around cut^2 (or marked far from the origin) take
-// the exact FP64 test, so the decisions are those of within_cut (the host
-// sizes the band above the FP32 rounding of points within R of the origin).
-// The FP32 decisions of a batch are branch-free; the exact test sits behind
-// one wave-uniform branch that a batch takes only when some lane has a
-// candidate in the band.  List slots are 32-bit element offsets from the
-// point's first chunk (the host keeps K * nf below 2^31).  The nine rows
-// are walked in a rolled loop with the next row's three cell ranges loaded
-// ahead: against nine unrolled rows with all ranges loaded up front, this
-// keeps the kernel under 128 VGPRs and a tenth of the code size, and builds
-// the lists 20 % faster (256k points: 153 vs 191 us).
-template <bool UNIF, int KIND, class PosT, int L, bool PRE, bool CODED = false>
-__device__ __forceinline__ int walk_list_lanes(const ListArgs& a, const PosT* __restrict__ B,
-                                               const float4* __restrict__ Bf, const int2* __restrict__ cells,
-                                               double x, double y, double z, float4 xf, double hA, int self,
-                                               int* __restrict__ out, int K, int q)
+// Squared distances, in units, around a cut of `cut` units between which the
+// FP64 test decides.  slack bounds the error of the distance (rounded FP32
+// coordinates and one unit of quantisation on three axes), err the rounding
+// of the FP32 square.  on = false: the FP64 test always.
+__host__ __device__ inline void cut_band(double cut, bool on, float slack, float err, float& lo, float& hi)
 {
-    const GridGeom& g = a.grid;
-    const double cut_u = KIND == kSolid ? 2.0 * hA : 2.0 * fmax(hA, KIND == kDummy ? a.hd : a.hf);
-    const unsigned cstride = (unsigned)a.nf * (unsigned)kChunk;
-    const Stencil st = make_stencil(g, x, y, z);
-    // row k's three cell ranges, loaded one row ahead of the walk
-    const auto row_load = [&](int k, int2* c) {
-        const int dz = k / 3 - 1, dy = k % 3 - 1;
-        const bool row_ok = dz >= st.loz && dz <= st.hiz && dy >= st.loy && dy <= st.hiy;
-        const int row = (st.cz + dz) * g.ny * g.nx + (st.cy + dy) * g.nx + st.cx;
-#pragma unroll
-        for (int dx = -1; dx <= 1; dx++) {
-            const bool ok = row_ok && dx >= st.lox && dx <= st.hix;
-            const int2 v = cells[ok ? row + dx : 0];
-            c[dx + 1] = ok ? v : make_int2(-1, -1);
-        }
-    };
-    int2 nxt[3];
-    row_load(0, nxt);
-    // this lane's L-bit window of a ballot: the 32-bit half holding the
-    // group, then a bit-field extract at the group's offset in that half
-    const int lane = threadIdx.x & 63;
-    const unsigned goff = (unsigned)((lane - q) & 31);
-    const bool hi_half = lane >= 32;
-    // a point far from the origin takes the exact test for every candidate
-    const float c2_u = (float)(cut_u * cut_u);
-    const float band_u = PRE && xf.w != 0.f ? INFINITY : a.band * c2_u;
-    int count = 0;
-#pragma unroll 1
-    for (int k = 0; k < 9; k++) {
-        const int2 cur[3] = {nxt[0], nxt[1], nxt[2]};
-        if (k < 8) row_load(k + 1, nxt);
-        int s0 = -1, e = -1;
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            if (cur[c].x != -1) {
-                if (s0 < 0) s0 = cur[c].x;
-                e = cur[c].y;
-            }
-        }
-        if (s0 < 0) { s0 = 0; e = 0; }
-        // coded lists: a slot's x-cell in the row is -1 below b0, 0 below b1, +1 above
-        const int b0 = cur[0].x != -1 ? cur[0].y : s0;
-        const int b1 = cur[1].x != -1 ? cur[1].y : b0;
-        const int rowcode = ((k / 3) << 4) | ((k % 3) << 2);  // (dz + 1) << 4 | (dy + 1) << 2
-        for (int j0 = s0; j0 < e; j0 += L * kLaneAhead) {
-            double qx[kLaneAhead], qy[kLaneAhead], qz[kLaneAhead];
-            float4 qf[kLaneAhead];
-#pragma unroll
-            for (int u = 0; u < kLaneAhead; u++) {
-                const unsigned jj = (unsigned)min(j0 + u * L + q, e - 1);
-                if (PRE) {
-                    qf[u] = Bf[jj];
-                } else {
-                    const PosT* b = B + jj;
-                    qx[u] = b->x; qy[u] = b->y; qz[u] = b->z;
-                }
-            }
-            bool hit[kLaneAhead];
-            double cutv[kLaneAhead];
-            bool need_any = false;
-            bool need[kLaneAhead];
-#pragma unroll
-            for (int u = 0; u < kLaneAhead; u++) {
-                const int j = j0 + u * L + q;
-                // bitwise, not short-circuit, operators: no branches per candidate
-                const bool valid = (j < e) & !(KIND == kFluid && j == self);
-                double cut = cut_u;
-                if (!UNIF && KIND != kSolid) {
-                    const int jc = min(j, e - 1);
-                    const double hB =
-                        KIND == kDummy ? a.phases[a.dphase[jc]].h : a.phases[phase_bits(a.V[jc].w)].h;
-                    cut = 2.0 * fmax(hA, hB);
-                }
-                cutv[u] = cut;
-                if (PRE) {
-                    const float c2 = UNIF || KIND == kSolid ? c2_u : (float)(cut * cut);
-                    const float band = UNIF || KIND == kSolid ? band_u : (xf.w != 0.f ? INFINITY : a.band * c2);
-                    const float fx = xf.x - qf[u].x, fy = xf.y - qf[u].y, fz = xf.z - qf[u].z;
-                    const float d2 = fx * fx + fy * fy + fz * fz;
-                    need[u] = valid & ((qf[u].w != 0.f) | (fabsf(d2 - c2) <= band));
-                    hit[u] = valid & (d2 < c2);
-                    need_any |= need[u];
-                } else {
-                    hit[u] = valid & within_cut(cut, x - qx[u], y - qy[u], z - qz[u]);
-                }
-            }
-            if (PRE && __ballot(need_any) != 0ull) {
-#pragma unroll
-                for (int u = 0; u < kLaneAhead; u++) {
-                    if (need[u]) {
-                        const PosT* b = B + (unsigned)(j0 + u * L + q);
-                        hit[u] = within_cut(cutv[u], x - b->x, y - b->y, z - b->z);
-                    }
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < kLaneAhead; u++) {
-                const unsigned long long bal = __ballot(hit[u]);
-                const unsigned half = hi_half ? (unsigned)(bal >> 32) : (unsigned)bal;
-                const unsigned gm = __builtin_amdgcn_ubfe(half, goff, L);
-                const int kk = count + __popc(gm & ((1u << q) - 1u));
-                const int j = j0 + u * L + q;
-                if (hit[u] & (kk < K))
-                    out[(unsigned)(kk >> 3) * cstride + (unsigned)(kk & (kChunk - 1))] =
-                        CODED ? j | (rowcode | (j >= b0) + (j >= b1)) << kCodeShift : j;
-                count += __popc(gm);
-            }
-        }
-    }
-    return count;
+    const double s = slack, l = cut - s, h = cut + s;
+    lo = on && l > 0.0 ? (float)(l * l * (1.0 - 1e-6) - err) : -INFINITY;
+    hi = on ? (float)(h * h * (1.0 + 1e-6) + err) : INFINITY;
 }
 
-template <bool UNIF, int LANES, bool PRE, bool CODED>
-__global__ __launch_bounds__(kThreads) void k_build_lists(ListArgs a)
+__device__ __forceinline__ int rl(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ __forceinline__ int nth_bit(unsigned m, int n)
 {
-    const int gt = xcd_block() * kThreads + threadIdx.x;
-    const int i = gt / LANES, q = gt % LANES;
-    if (i >= a.nf) return;  // uniform over a lane group
-    const FluidPos p = a.P[i];
-    const float4 pf = PRE ? a.Pf[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const double h = UNIF ? a.hf : a.phases[phase_bits(a.V[i].w)].h;
-    int* of = a.nbr_ff + (size_t)i * kChunk;
-    const int c1 = LANES == 1 ? walk_list<UNIF, kFluid, FluidPos, CODED>(a, a.P, a.cells, p.x, p.y, p.z, h, i, of,
-                                                                          a.K_ff)
-                              : walk_list_lanes<UNIF, kFluid, FluidPos, LANES, PRE, CODED>(
-                                    a, a.P, a.Pf, a.cells, p.x, p.y, p.z, pf, h, i, of, a.K_ff, q);
-    int c2 = 0;
-    if (a.nd > 0 && a.dummy_near[cell_hash(a.grid, p.x, p.y, p.z)]) {
-        int* od = a.nbr_fd + (size_t)i * kChunk;
-        c2 = LANES == 1 ? walk_list<UNIF, kDummy>(a, a.DP, a.dcells, p.x, p.y, p.z, h, -1, od, a.K_fd)
-                        : walk_list_lanes<UNIF, kDummy, DummyPos, LANES, PRE>(
-                              a, a.DP, a.DPf, a.dcells, p.x, p.y, p.z, pf, h, -1, od, a.K_fd, q);
+    for (; n > 0; n--) m &= m - 1;
+    return __ffs(m) - 1;
+}
+
+// List build.  A wave takes G consecutive slots and, of these, the particles
+// that share a stencil centre together (a set): their nine runs of candidate
+// slots, laid end to end, are loaded 64 at a time, one candidate a lane, and
+// tested against one particle after the other.  A ballot is the hit mask:
+// its population advances the particle's count, and the lanes of the mask
+// store their slots at the count plus their rank, so the list keeps the
+// walk's order.
+//
+// Coordinates are taken relative to the middle of the centre cell, and a test
+// is three fused multiply-adds and two compares:
+//   |b - a|^2 < c^2  <=>  |b|^2 - 2 a . b < c^2 - |a|^2,
+// with -2 a, the right-hand sides of the band's two ends and the count read
+// from LDS as a broadcast.  The cell of a particle in the grid is half a cell
+// wide about that point; a set is made of particles within three quarters of
+// the largest edge of it on every axis, |a| <= A, and takes plain tests.  A
+// pair near the cut has |b| <= B = A + c, and its test at most three roundings
+// of 2^-24 B^2, three of B^2 + 2 A B, three of A^2 and one of A^2 + c^2: half
+// the bound that list_error takes.  Candidates farther off (outside the
+// grid, 15 cells at most, or out as FixGeom has it) are off by less than
+// 1e-6 of |b|^2 and clear of the cut by more.
+// Any other particle is a set by itself about its own position, and also
+// takes the exact test against far candidates; one that is out takes no
+// other.  A particle that has left the grid so costs no one else an exact
+// test: with all pairs of its cell on it, the build of 18k particles took 55
+// us instead of 46 once some had run over the walls.
+// Candidates in the band take the exact test behind a scalar branch; so do
+// all pairs of a set whose own slots are not in its centre row.
+//
+// Bound by VALU issue.  Lanes that each walked candidates of their own
+// particle took 40 instructions per 64 candidates, and seven times the loads.
+constexpr float kListSlack = 64.0f;  // of the distance: 2 (8 + 8 + 1) sqrt(3), for coordinates below 2^28
+// Error bound of a plain test of reach A (per axis) and cut c.
+inline float list_error(double reach, double c)
+{
+    const double A = sqrt(3.0) * reach, B = A + c;
+    return (float)((3.0 * B * B + 3.0 * (B * B + 2.0 * A * B) + 4.0 * A * A + c * c) / 8388608.0);
+}
+
+// The nine runs of a stencil laid end to end: run r ends before e_r and its
+// slots are their places plus o_r.
+struct Runs {
+    int e0, e1, e2, e3, e4, e5, e6, e7, o0, o1, o2, o3, o4, o5, o6, o7, o8;
+};
+__device__ __forceinline__ int run_slot(const Runs r, int t)
+{
+    int o = t < r.e7 ? r.o7 : r.o8;
+    o = t < r.e6 ? r.o6 : o;
+    o = t < r.e5 ? r.o5 : o;
+    o = t < r.e4 ? r.o4 : o;
+    o = t < r.e3 ? r.o3 : o;
+    o = t < r.e2 ? r.o2 : o;
+    o = t < r.e1 ? r.o1 : o;
+    o = t < r.e0 ? r.o0 : o;
+    return t + o;
+}
+
+// The particles of a set in LDS.  UNIF scenes: w and hi are the band's ends
+// less |a|^2; otherwise w = |a|^2 and lo, hi the band of the own cut.
+constexpr int kListBatch = 4;  // particles tested together
+template <int G>
+struct alignas(16) ListOwn {
+    float4 a[G + kListBatch];  // -2 a, w
+    float hi[G + kListBatch], lo[G + kListBatch];
+    int count[G + kListBatch], base[G + kListBatch];  // list entries so far; bytes from slot w0's first entry to its own
+    int self[G + kListBatch];                         // slots behind the set's first
+};
+
+// What a wave lists against: the fluid's slots, or the dummies'.
+struct ListSet {
+    bool dummy;
+    const char* P;    // 32-byte records that begin with the FP64 position
+    const float4* A;  // fixed-point positions
+    const int2* cells;
+    float lo, hi;     // cut band of uniform scenes
+    double cut;       // and their cut
+    int* lists;
+    int K;
+};
+
+constexpr float kFixMiss = 1e38f;  // a square beyond every band but the open one
+
+// The fixed-point coordinate of the middle of cell c of an axis.
+__device__ __forceinline__ int cell_middle(int c, unsigned long long step)
+{
+    return (int)(((unsigned long long)c * step + step / 2) >> 20);
+}
+
+template <bool UNIF, int G>
+__device__ __forceinline__ void walk_sets(const ListArgs& a, const ListSet& v, int w0, unsigned live, const float4& r,
+                                          bool plain, int cell, int cell_x, int cell_y, int cell_z, double h,
+                                          int& count, bool& far_pair, ListOwn<G>& own)
+{
+    constexpr int NB = kListBatch;
+    const GridGeom& g = a.grid;
+    const int lane = threadIdx.x & 63;
+    const int qx = __float_as_int(r.x), qy = __float_as_int(r.y), qz = __float_as_int(r.z);
+    const unsigned plains = (unsigned)__ballot(plain), far_set = (unsigned)__ballot(r.w < 0.0f) & live;
+    const int K = v.K;
+    char* const out = reinterpret_cast<char*>(v.lists + list_entry(w0, 0, K));
+    unsigned fars = 0;
+    for (unsigned left = live; left;) {
+        const int kf = __ffs(left) - 1;
+        const bool inner = plains >> kf & 1u;
+        const unsigned set = inner ? (unsigned)__ballot(cell == rl(cell, kf)) & left & plains : 1u << kf;
+        left &= ~set;
+        const int ns = __popc(set);
+        const int cx = rl(cell_x, kf), cy = rl(cell_y, kf), cz = rl(cell_z, kf);
+        const int rx = inner ? cell_middle(cx, a.stepx) : rl(qx, kf), ry = inner ? cell_middle(cy, a.stepy) : rl(qy, kf),
+                  rz = inner ? cell_middle(cz, a.stepz) : rl(qz, kf);
+        // the set's particles in order, padded to whole batches with ones that hit nothing
+        const int place = __popc(set & ((1u << (lane & 31)) - 1u));
+        if (lane < NB) {
+            own.a[ns + lane] = make_float4(0.f, 0.f, 0.f, UNIF ? -INFINITY : INFINITY);
+            own.hi[ns + lane] = own.lo[ns + lane] = -INFINITY;
+            own.count[ns + lane] = own.base[ns + lane] = own.self[ns + lane] = 0;
+        }
+        if (lane < G && (set >> lane & 1u)) {
+            const float x = (float)(qx - rx), y = (float)(qy - ry), z = (float)(qz - rz);
+            const float n2 = x * x + y * y + z * z;
+            float lo = v.lo, hi = v.hi, w = n2;
+            if (!UNIF) cut_band(2.0 * h * a.inv, a.prefilter != 0, kListSlack, a.err, lo, hi);
+            if (r.w < 0.0f) {  // every candidate in the band, or none
+                lo = -INFINITY;
+                hi = r.w == -1.0f ? INFINITY : -INFINITY;
+                w = r.w == -1.0f ? kFixMiss : INFINITY;
+            }
+            own.a[place] = make_float4(-2.0f * x, -2.0f * y, -2.0f * z, UNIF ? lo - n2 : w);
+            own.hi[place] = UNIF ? hi - n2 : hi;
+            own.lo[place] = lo;
+            own.self[place] = lane - kf;
+            own.count[place] = 0;
+            own.base[place] = (int)(4 * (list_entry(w0 + lane, 0, K) - list_entry(w0, 0, K)));
+        }
+        // row r's run of slots in lane r, its place among the packed candidates
+        int rs = 0, len = 0;
+        if (lane < 9) {
+            const int z = cz + lane / 3 - 1, y = cy + lane % 3 - 1;
+            if (z >= 0 && z < g.nz && y >= 0 && y < g.ny) {
+                const int2* row = v.cells + ((size_t)z * g.ny + y) * g.nx;
+                const int2 none = make_int2(-1, -1);
+                const int2 c0 = cx > 0 ? row[cx - 1] : none, c1 = row[cx], c2 = cx < g.nx - 1 ? row[cx + 1] : none;
+                const int s = c0.x != -1 ? c0.x : c1.x != -1 ? c1.x : c2.x;
+                if (s != -1) {
+                    rs = s;
+                    len = (c2.x != -1 ? c2.y : c1.x != -1 ? c1.y : c0.y) - s;
+                }
+            }
+        }
+        int inc = len;
+#pragma unroll
+        for (int d = 1; d < 16; d <<= 1) {
+            const int t = __shfl_up(inc, d, 16);
+            if ((lane & 15) >= d) inc += t;
+        }
+        const int total = rl(inc, 8);
+        const int shift = rs - (inc - len);  // slot - place in the run
+        const Runs runs{rl(inc, 0), rl(inc, 1), rl(inc, 2), rl(inc, 3), rl(inc, 4), rl(inc, 5), rl(inc, 6), rl(inc, 7),
+                        rl(shift, 0), rl(shift, 1), rl(shift, 2), rl(shift, 3), rl(shift, 4), rl(shift, 5),
+                        rl(shift, 6), rl(shift, 7), rl(shift, 8)};
+        // place of the set's first slot among the fluid's candidates; its
+        // slots lie in the centre row but for some far points
+        const int self0 = w0 + kf - runs.o4;
+        const bool regular = v.dummy || (self0 >= runs.e3 && self0 + (31 - __clz((int)set)) - kf < runs.e4);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        int j_next = 0;
+        float4 q_next = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (total > 0) {
+            j_next = run_slot(runs, min(lane, total - 1));
+            q_next = v.A[j_next];
+        }
+        for (int t0 = 0; t0 < total; t0 += 64) {
+            const int j = j_next;
+            const float4 q = q_next;
+            if (t0 + 64 < total) {
+                j_next = run_slot(runs, min(t0 + 64 + lane, total - 1));
+                q_next = v.A[j_next];
+            }
+            const bool in = t0 + lane < total;
+            const float x = (float)(__float_as_int(q.x) - rx), y = (float)(__float_as_int(q.y) - ry),
+                        z = (float)(__float_as_int(q.z) - rz);
+            const float n2 = in ? (q.w == -2.0f ? kFixMiss : x * x + y * y + z * z) : INFINITY;
+            const unsigned long long inm = __ballot(in), farm = __ballot(q.w < 0.0f) & inm;
+            const unsigned long long cold = regular ? (inner ? __ballot(q.w == -1.0f) & inm : farm) : inm;
+            float lo_j = 0.f, hi_j = 0.f;
+            double hB = 0.0;
+            if (!UNIF) {
+                hB = a.phases[v.dummy ? a.dphase[j] : phase_bits(a.V[j].w)].h;
+                cut_band(2.0 * hB * a.inv, a.prefilter != 0, kListSlack, a.err, lo_j, hi_j);
+            }
+            const int s0 = self0 - t0;  // the set's own slots among these candidates
+            const bool owns = !v.dummy && s0 > -G && s0 < 64;
+            for (int p = 0; p < ns; p += NB) {
+                const float4 hi4 = *reinterpret_cast<const float4*>(&own.hi[p]);
+                const float hi[NB] = {hi4.x, hi4.y, hi4.z, hi4.w};
+                float lo[NB] = {0.f, 0.f, 0.f, 0.f};
+                if (!UNIF) {
+                    const float4 lo4 = *reinterpret_cast<const float4*>(&own.lo[p]);
+                    lo[0] = lo4.x; lo[1] = lo4.y; lo[2] = lo4.z; lo[3] = lo4.w;
+                }
+                unsigned long long hit[NB], near[NB], any = cold;
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    const float4 s = own.a[p + b];
+                    float d = fmaf(s.x, x, fmaf(s.y, y, fmaf(s.z, z, n2)));
+                    if (UNIF) {
+                        hit[b] = __ballot(d < s.w);
+                        near[b] = __ballot(d < hi[b]) & ~hit[b];
+                    } else {
+                        d += s.w;
+                        hit[b] = __ballot(d < fmaxf(lo[b], lo_j));
+                        near[b] = __ballot(d < fmaxf(hi[b], hi_j)) & ~hit[b];
+                    }
+                    any |= near[b];
+                }
+                if (owns) {
+                    const int4 o4 = *reinterpret_cast<const int4*>(&own.self[p]);
+                    const int o[NB] = {rl(o4.x, 0), rl(o4.y, 0), rl(o4.z, 0), rl(o4.w, 0)};
+#pragma unroll
+                    for (int b = 0; b < NB; b++)
+                        if ((unsigned)(s0 + o[b]) < 64u) hit[b] &= ~(1ull << (s0 + o[b]));
+                }
+                if (__builtin_expect(any != 0, 0)) {
+#pragma unroll 1
+                    for (int b = 0; b < NB; b++) {
+                        if (p + b >= ns) break;
+                        const int k = nth_bit(set, p + b);
+                        const unsigned long long hb = b == 0 ? hit[0] : b == 1 ? hit[1] : b == 2 ? hit[2] : hit[3];
+                        const unsigned long long nb = b == 0 ? near[0] : b == 1 ? near[1] : b == 2 ? near[2] : near[3];
+                        const unsigned long long m = nb | cold;
+                        bool ok = false;
+                        if (m >> lane & 1ull) {
+                            const FluidPos f = a.P[w0 + k];
+                            const double* o = reinterpret_cast<const double*>(v.P + (size_t)j * sizeof(FluidPos));
+                            const double cut = UNIF ? v.cut : 2.0 * fmax(a.phases[phase_bits(a.V[w0 + k].w)].h, hB);
+                            ok = (v.dummy || j != w0 + k) && within_cut(cut, f.x - o[0], f.y - o[1], f.z - o[2]);
+                        }
+                        const unsigned long long r = (hb & ~m) | __ballot(ok);
+                        if ((far_set >> k & 1u) || (r & farm)) fars |= 1u << k;
+                        hit[0] = b == 0 ? r : hit[0];
+                        hit[1] = b == 1 ? r : hit[1];
+                        hit[2] = b == 2 ? r : hit[2];
+                        hit[3] = b == 3 ? r : hit[3];
+                    }
+                }
+                const int4 n4 = *reinterpret_cast<const int4*>(&own.count[p]), b4 = *reinterpret_cast<const int4*>(&own.base[p]);
+                const int cnt[NB] = {n4.x, n4.y, n4.z, n4.w}, base[NB] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    // a full list goes on behind its end, in the rows of the
+                    // next slots: such lists are never used (the overflow
+                    // grows them and repeats the search), and the allocation
+                    // ends with room for one batch of candidates
+                    const unsigned e = __builtin_amdgcn_mbcnt_hi(
+                        (unsigned)(hit[b] >> 32),
+                        __builtin_amdgcn_mbcnt_lo((unsigned)hit[b], min((unsigned)cnt[b], (unsigned)K)));
+                    if (__builtin_expect(__builtin_amdgcn_inverse_ballot_w64(hit[b]), 1))
+                        *reinterpret_cast<int*>(out + ((unsigned)base[b] + 4u * e +
+                                                       (e >> 3) * (4u * kChunk * (kListRows - 1)))) = j;
+                }
+                if (lane == 0)
+                    *reinterpret_cast<int4*>(&own.count[p]) =
+                        make_int4(cnt[0] + __popcll(hit[0]), cnt[1] + __popcll(hit[1]), cnt[2] + __popcll(hit[2]),
+                                  cnt[3] + __popcll(hit[3]));
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (lane < G && (set >> lane & 1u)) count = own.count[place];
     }
-    if (q != 0) return;
-    a.cnt_ff[i] = c1;
-    a.cnt_fd[i] = c2;
-    if (CODED) {
-        const Stencil st = make_stencil(a.grid, p.x, p.y, p.z);
-        a.pcen[i] = pack_cell(st.cx, st.cy, st.cz);
+    far_pair = fars >> (lane & 31) & 1u;
+}
+
+// Fluid-fluid and fluid-dummy lists of the reference
+// (SPHNeighborSearchKernel.cu:6-228), per_wave particles a wave, G at a time.
+template <bool UNIF, int G>
+__global__ __launch_bounds__(kThreads, 6) void k_build_lists(ListArgs a, int per_wave)
+{
+    static_assert(G <= 32, "the sets are 32-bit masks");
+    static_assert(kListBatch == 4, "the exact test names the hits of a batch");
+    static_assert(sizeof(FluidPos) == sizeof(DummyPos), "one stride for both position records");
+    __shared__ ListOwn<G> own_s[kThreads / 64];
+    const GridGeom& g = a.grid;
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const long long first = ((long long)xcd_block_spread<16>() * (kThreads / 64) + wv) * per_wave;
+    for (int sub = 0; sub < per_wave && first + sub < a.nf; sub += G) {
+        const int w0 = (int)first + sub;
+        const int n = min(G, a.nf - w0);
+        const int i = w0 + min(lane, n - 1);
+        const float4 r = a.A[i];
+        const bool far = r.w < 0.0f;
+        const uint32_t key = a.skey[i];
+        // the stencil centre: the hashed cell, but for far points
+        int cell = (int)key;
+        if (__builtin_expect(__ballot(far) != 0, 0)) {
+            const FluidPos p = a.P[i];
+            const Stencil st = make_stencil(g, p.x, p.y, p.z);
+            cell = far ? (st.cz * g.ny + st.cy) * g.nx + st.cx : cell;
+        }
+        const int nxy = g.nx * g.ny;
+        const int cz = cell / nxy, cy = (cell - cz * nxy) / g.nx, cx = cell - cz * nxy - cy * g.nx;
+        const double h = UNIF ? a.hf : a.phases[phase_bits(a.V[i].w)].h;
+        const float x = (float)(__float_as_int(r.x) - cell_middle(cx, a.stepx)),
+                    y = (float)(__float_as_int(r.y) - cell_middle(cy, a.stepy)),
+                    z = (float)(__float_as_int(r.z) - cell_middle(cz, a.stepz));
+        const bool plain = !far && fmaxf(fmaxf(fabsf(x), fabsf(y)), fabsf(z)) < a.reach;
+        const unsigned live = n == 32 ? ~0u : (1u << n) - 1u;
+        unsigned dnear = 0;
+        if (a.nd > 0) dnear = (unsigned)__ballot((long long)key < a.numGrids && a.dummy_near[key] != 0) & live;
+#pragma unroll 1
+        // both kinds of neighbour, or those of the block
+        for (int kind = blockIdx.y; kind < 2; kind += gridDim.y) {
+            const bool d = kind != 0;
+            const ListSet v{d,
+                            d ? reinterpret_cast<const char*>(a.DP) : reinterpret_cast<const char*>(a.P),
+                            d ? a.DA : a.A,
+                            d ? a.dcells : a.cells,
+                            d ? a.lo_d : a.lo_f,
+                            d ? a.hi_d : a.hi_f,
+                            d ? 2.0 * fmax(a.hf, a.hd) : 2.0 * a.hf,
+                            d ? a.nbr_fd : a.nbr_ff,
+                            d ? a.K_fd : a.K_ff};
+            int count = 0;  // lane k: particle w0 + k
+            bool far_pair = false;
+            walk_sets<UNIF, G>(a, v, w0, d ? dnear : live, r, plain, cell, cx, cy, cz, h, count, far_pair,
+                               own_s[wv]);
+            if (lane < n) {
+                (d ? a.cnt_fd : a.cnt_ff)[i] = count | (far_pair ? kFarBit : 0);
+                if (count > v.K) atomicMax(&a.maxcount[kind], count);
+            }
+        }
     }
-    if (c1 > a.K_ff) atomicMax(&a.maxcount[0], c1);
-    if (c2 > a.K_fd) atomicMax(&a.maxcount[1], c2);
 }
 
 // Fluid -> coupled-ball lists over the balls sorted into the fluid grid.
@@ -709,8 +920,7 @@ __global__ __launch_bounds__(kThreads) void k_build_fs_lists(ListArgs a)
     if (i >= a.nf) return;
     const FluidPos p = a.P[i];
     const double h = a.phases[phase_bits(a.V[i].w)].h;
-    const int c = walk_list<true, kSolid>(a, a.SP, a.scells, p.x, p.y, p.z, h, -1, a.nbr_fs + (size_t)i * kChunk,
-                                          a.K_fs);
+    const int c = walk_solids(a, p.x, p.y, p.z, h, a.nbr_fs + (size_t)i * kChunk, a.K_fs);
     a.cnt_fs[i] = c;
     if (c > a.K_fs) atomicMax(&a.maxcount[2], c);
 }
@@ -758,20 +968,19 @@ __device__ __forceinline__ void for_chunks(const int* __restrict__ list, int cnt
     }
 }
 
-// for_chunks in two phases per batch: every entry's records are gathered
-// (load) before any is used (use), so kBatch independent gathers are in
-// flight per lane.  A chunk's eight indices are read at once; batches of
-// kBatch entries follow in order.  Same entries, same order as for_chunks.
-template <int LANES, class LoadF, class UseF>
-__device__ __forceinline__ void for_chunks_gathered(const int* __restrict__ list, int cnt, int K, int nf, int i, int q,
-                                                    int safe, LoadF&& load, UseF&& use)
+// One lane over a whole row, in order, in two phases per batch: every
+// entry's records are gathered (load) before any is used (use), so kBatch
+// independent gathers are in flight.  Eight indices are read at once; batches
+// of kBatch entries follow in order.
+template <class LoadF, class UseF>
+__device__ __forceinline__ void for_row(const int* __restrict__ list, int cnt, int K, int i, int safe, LoadF&& load,
+                                        UseF&& use)
 {
-    const int n = min(cnt, K);
-    const int* L = list + (size_t)i * kChunk;
-    const size_t cs = (size_t)nf * kChunk;
-    for (int c = q; c * kChunk < n; c += LANES) {
+    const int n = min(list_count(cnt), K);
+    const int* L = list + list_entry(i, 0, K);
+    for (int c = 0; c * kChunk < n; c++) {
         const int base = c * kChunk;
-        const int4* src = reinterpret_cast<const int4*>(L + (size_t)c * cs);
+        const int4* src = reinterpret_cast<const int4*>(L + c * kListStride);
         const int4 lo = src[0];
         const int4 hi = base + 4 < n ? src[1] : make_int4(safe, safe, safe, safe);
         const int jall[kChunk] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
@@ -803,6 +1012,10 @@ struct DummyRec {
     DummyPos D;
     float4 V;
 };
+struct DummyFix {
+    float4 A, B;
+    float2 C;
+};
 
 // Sum over the LANES lanes of a particle (a fixed butterfly order).
 template <int LANES, class T>
@@ -824,18 +1037,17 @@ __device__ __forceinline__ T ld_at(const T* __restrict__ base, int j)
 __device__ __forceinline__ GRec ld_grec(const float4* __restrict__ base, int half, int j)
 {
     const float4 a = ld_at(base, j), b = ld_at(base + half, j);
-    return GRec{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    return GRec{__float_as_int(a.x), __float_as_int(a.y), __float_as_int(a.z), a.w, b.x, b.y, b.z, b.w};
 }
 
 // Per-particle values of a pair pass.
 struct PairSelf {
-    double x, y, z;
+    double x, y, z;       // FP64 records only
+    int qx, qy, qz;       // gather records only
     float vx, vy, vz, w;  // w: phase bits
     float rho, p, inv_rho;
     Phase ph;
     GradK gff, gfd;  // uniform scenes: kernel constants of fluid and dummy pairs
-    float ox, oy, oz;     // gather records: offset from the stencil centre's origin
-    float csx, csy, csz;  // cell size
 };
 
 template <bool UNIF>
@@ -845,6 +1057,7 @@ __device__ __forceinline__ PairSelf pair_self(const SphArgs& a, int i)
     const float4 Vi = a.V[i];
     PairSelf s;
     s.x = Pi.x; s.y = Pi.y; s.z = Pi.z;
+    s.qx = s.qy = s.qz = 0;
     s.vx = Vi.x; s.vy = Vi.y; s.vz = Vi.z; s.w = Vi.w;
     s.ph = UNIF ? a.phf : a.phases[phase_bits(Vi.w)];
     s.rho = Pi.rho; s.p = Pi.p;
@@ -853,57 +1066,116 @@ __device__ __forceinline__ PairSelf pair_self(const SphArgs& a, int i)
         s.gff = grad_k(0.5f * (s.ph.hf + a.phf.hf));
         s.gfd = grad_k(0.5f * (s.ph.hf + a.phd.hf));
     }
-    if (a.GRin) {
-        double x0, y0, z0;
-        cell_origin(a.grid, a.pcen[i], x0, y0, z0);
-        s.ox = (float)(s.x - x0); s.oy = (float)(s.y - y0); s.oz = (float)(s.z - z0);
-        s.csx = (float)a.grid.cx; s.csy = (float)a.grid.cy; s.csz = (float)a.grid.cz;
-    }
+    return s;
+}
+// The same from the gather records (uniform scenes).
+__device__ __forceinline__ PairSelf pair_self_rec(const SphArgs& a, int i)
+{
+    const GRec r = ld_grec(a.GRin, a.nf, i);
+    PairSelf s;
+    s.x = s.y = s.z = 0.0;
+    s.qx = r.qx; s.qy = r.qy; s.qz = r.qz;
+    s.vx = r.vx; s.vy = r.vy; s.vz = r.vz; s.w = 0.f;
+    s.ph = a.phf;
+    s.rho = r.rho; s.p = r.p;
+    s.inv_rho = 1.0f / s.rho;
+    s.gff = GradK{};
+    s.gfd = GradK{};
     return s;
 }
 
-// momentum_ff on a gather record; code holds the neighbour's cell relative
-// to the stencil centre, 2 bits (offset + 1) per axis.
-__device__ __forceinline__ void momentum_ff_g(const SphArgs& a, const PairSelf& s, const GRec& R, int code, bool valid,
-                                              float& ax, float& ay, float& az)
+// Pair terms on gather records.  Distances stay in units of the fixed-point
+// grid; the constant factors of a pass (unit, kernel constant, mass, own
+// density, viscosity) are taken out of the sums and applied once per lane.
+// Entries past a list's end are the particle itself: zero distance and zero
+// velocity difference make every term an exact zero.
+struct PairDist {
+    float x, y, z, r, inv_r, t3;  // difference, distance, 1/distance, (1 - r/2h)^3
+};
+__device__ __forceinline__ PairDist pair_dist(int ax, int ay, int az, int bx, int by, int bz, float half_invh_u)
 {
-    const Phase& pj = a.phf;
-    const float dcx = (float)(code & 3) - 1.0f, dcy = (float)((code >> 2) & 3) - 1.0f, dcz = (float)(code >> 4) - 1.0f;
-    const float rx = (s.ox - R.ox) - dcx * s.csx, ry = (s.oy - R.oy) - dcy * s.csy, rz = (s.oz - R.oz) - dcz * s.csz;
-    const float r2 = rx * rx + ry * ry + rz * rz;
-    const float inv_r = (r2 < 1.e-20f) ? 0.0f : rsq(r2);
-    const float r = r2 * inv_r;
-    const float g = grad_factor(r, s.gff);
-    const float f = valid ? g : 0.0f;
-    const float dvx = s.vx - R.vx, dvy = s.vy - R.vy, dvz = s.vz - R.vz;
-    const float dU = -(dvx * rx + dvy * ry + dvz * rz) * inv_r;
-    const float cbar = 0.5f * (s.ph.c + pj.c);
-    const float beta = fminf(3.0f * fmaxf(dU, 0.0f), cbar);
-    const float Ps = 0.5f * (s.p + R.p) + 0.25f * beta * (s.rho + R.rho) * dU;
-    const float fm = f * (pj.m * s.inv_rho) * rcp(R.rho);
-    const float kp = -2.0f * Ps * fm;
-    const float kv = (s.ph.nu + pj.nu) * r * fm;
-    ax += kp * rx + kv * dvx;
-    ay += kp * ry + kv * dvy;
-    az += kp * rz + kv * dvz;
+    PairDist d;
+    d.x = (float)(ax - bx); d.y = (float)(ay - by); d.z = (float)(az - bz);
+    const float r2 = d.x * d.x + d.y * d.y + d.z * d.z;
+    // distances are whole units: only zero is below 1
+    d.inv_r = rsq(fmaxf(r2, 0.25f));
+    d.r = r2 * d.inv_r;
+    const float t = fmaxf(1.0f - d.r * half_invh_u, 0.0f);
+    d.t3 = t * t * t;
+    return d;
 }
 
-// continuity_ff on a gather record.
-__device__ __forceinline__ float continuity_ff_g(const SphArgs& a, const PairSelf& s, const GRec& R, int code,
-                                                 bool valid)
+// Sums of momentum_ff over fluid neighbours: P: sum of 2 P* t^3 / rho_j times
+// the difference, V: sum of r t^3 / rho_j times the velocity difference.
+struct MomentumSums {
+    float px, py, pz, vx, vy, vz;
+};
+__device__ __forceinline__ void momentum_ff_g(const PairSelf& s, const GRec& R, float half_invh_u, float half_c,
+                                              MomentumSums& m)
 {
-    const Phase& pj = a.phf;
-    const float dcx = (float)(code & 3) - 1.0f, dcy = (float)((code >> 2) & 3) - 1.0f, dcz = (float)(code >> 4) - 1.0f;
-    const float rx = (s.ox - R.ox) - dcx * s.csx, ry = (s.oy - R.oy) - dcy * s.csy, rz = (s.oz - R.oz) - dcz * s.csz;
-    const float r2 = rx * rx + ry * ry + rz * rz;
-    const float inv_r = (r2 < 1.e-20f) ? 0.0f : rsq(r2);
-    const float r = r2 * inv_r;
-    const float g = grad_factor(r, s.gff);
-    const float f = valid ? g : 0.0f;
-    const float cbar = 0.5f * (s.ph.c + pj.c);
-    const float dvr = (s.vx - R.vx) * rx + (s.vy - R.vy) * ry + (s.vz - R.vz) * rz;
-    const float q = (s.p - R.p) * r * rcp((s.rho + R.rho) * (0.5f * cbar));
-    return (0.5f * pj.m) * f * rcp(R.rho) * (dvr + q);
+    const PairDist d = pair_dist(s.qx, s.qy, s.qz, R.qx, R.qy, R.qz, half_invh_u);
+    const float dvx = s.vx - R.vx, dvy = s.vy - R.vy, dvz = s.vz - R.vz;
+    const float dU = -(dvx * d.x + dvy * d.y + dvz * d.z) * d.inv_r;
+    // beta / 2, beta = min(3 max(U_L - U_R, 0), c)
+    const float hb = __builtin_amdgcn_fmed3f(1.5f * dU, 0.0f, half_c);
+    const float Ps2 = (s.p + R.p) + hb * dU * (s.rho + R.rho);
+    const float w = d.t3 * rcp(R.rho);
+    const float kp = Ps2 * w, kv = d.r * w;
+    m.px += kp * d.x; m.py += kp * d.y; m.pz += kp * d.z;
+    m.vx += kv * dvx; m.vy += kv * dvy; m.vz += kv * dvz;
+}
+
+// Sum of continuity_ff over fluid neighbours without the factor
+// u coef m_j / 2: t^3 / rho_j [ dv . r + (P_L - P_R) r / (rho_bar c) ], over
+// one common denominator.
+__device__ __forceinline__ void continuity_ff_g(const PairSelf& s, const GRec& R, float half_invh_u, float half_c,
+                                                float rho_c, float& sum)
+{
+    const PairDist d = pair_dist(s.qx, s.qy, s.qz, R.qx, R.qy, R.qz, half_invh_u);
+    const float dvr = (s.vx - R.vx) * d.x + (s.vy - R.vy) * d.y + (s.vz - R.vz) * d.z;
+    const float rc = R.rho * half_c + rho_c;  // rho_bar c
+    const float num = dvr * rc + (s.p - R.p) * d.r;
+    sum += d.t3 * rcp(R.rho * rc) * num;
+}
+
+// momentum_fd and continuity_fd on records; a lane's entries past the end
+// count as out of reach.
+__device__ __forceinline__ PairDist dummy_dist(const SphArgs& a, const PairSelf& s, const DummyFix& R, bool valid,
+                                               float& PR, float& rhoj)
+{
+    PairDist d = pair_dist(s.qx, s.qy, s.qz, __float_as_int(R.A.x), __float_as_int(R.A.y), __float_as_int(R.A.z),
+                           a.fd_half_invh);
+    d.t3 = valid ? d.t3 : 0.0f;
+    const float grj = fmaxf(-(a.gx * d.x + a.gy * d.y + a.gz * d.z) * a.fix.u, 0.0f);
+    PR = s.p + s.rho * grj;
+    rhoj = dummy_rho(a, a.phd, PR);
+    return d;
+}
+__device__ __forceinline__ void momentum_fd_g(const SphArgs& a, const PairSelf& s, const DummyFix& R, bool valid,
+                                              MomentumSums& m)
+{
+    float PR, rhoj;
+    const PairDist d = dummy_dist(a, s, R, valid, PR, rhoj);
+    const float nx = R.B.x, ny = R.B.y, nz = R.B.z;
+    const float UL = -(nx * s.vx + ny * s.vy + nz * s.vz);
+    const float UR = -UL - 2.0f * (nx * R.B.w + ny * R.C.x + nz * R.C.y);
+    const float cbar = 0.5f * (s.ph.c + a.phd.c), rbar = 0.5f * (s.rho + rhoj);
+    const float beta = fminf(3.0f * fmaxf(UL - UR, 0.0f), cbar);
+    const float Ps2 = (s.p + PR) + beta * rbar * (UL - UR);
+    const float w = d.t3 * rcp(rhoj);
+    const float kp = Ps2 * w, kv = d.r * w;
+    m.px += kp * d.x; m.py += kp * d.y; m.pz += kp * d.z;
+    m.vx += kv * (s.vx - R.B.w); m.vy += kv * (s.vy - R.C.x); m.vz += kv * (s.vz - R.C.y);
+}
+__device__ __forceinline__ void continuity_fd_g(const SphArgs& a, const PairSelf& s, const DummyFix& R, bool valid,
+                                                float& sum)
+{
+    float PR, rhoj;
+    const PairDist d = dummy_dist(a, s, R, valid, PR, rhoj);
+    const float cbar = 0.5f * (s.ph.c + a.phd.c), rbar = 0.5f * (s.rho + rhoj);
+    const float t = (s.vx - R.B.w) * d.x + (s.vy - R.C.x) * d.y + (s.vz - R.C.y) * d.z +
+                    (s.p - PR) * d.r * rcp(rbar * cbar);
+    sum += d.t3 * rcp(rhoj) * t;
 }
 
 // One fluid neighbour's term of updateWCSPHAccelerationKernel
@@ -970,22 +1242,25 @@ __device__ __forceinline__ void momentum_fd(const SphArgs& a, const PairSelf& s,
     az += kp * rz + kv * (s.vz - DVj.z);
 }
 
-// Lane-group sum, coupled balls, gravity, half kick (:150-159) and, in the
-// first half, the drift (:161-170).
-template <bool FIRST, int LANES>
-__device__ __forceinline__ void momentum_finish(const SphArgs& a, const PairSelf& s, int i, int q, float ax, float ay,
-                                                float az)
+// Lane-group sum, coupled balls (their own instantiations: the ball terms
+// hold 30 more registers), gravity, half kick (:150-159) and, in the first
+// half, the drift (:161-170).
+template <bool FIRST, int LANES, bool BALLS>
+__device__ __forceinline__ void momentum_finish(const SphArgs& a, int i, int q, float ax, float ay, float az)
 {
     if (LANES > 1) {
         ax = lane_group_sum<LANES>(ax);
         ay = lane_group_sum<LANES>(ay);
         az = lane_group_sum<LANES>(az);
     }
-    if (a.ns > 0) {
+    if constexpr (BALLS) {
+        const FluidPos s = a.P[i];
+        const float4 v = a.V[i];
+        const Phase ph = a.phases[phase_bits(v.w)];
         float cx = 0.f, cy = 0.f, cz = 0.f;
         for_chunks<LANES>(a.nbr_fs, a.cnt_fs[i], a.K_fs, a.nf, i, q, 0, [&](int j, bool valid) {
             float3 ap, av, lv;
-            fs_momentum(a, s.ph, s.x, s.y, s.z, s.vx, s.vy, s.vz, s.rho, s.p, a.SP[j], a.SV[j], a.SW[j], ap, av, lv);
+            fs_momentum(a, ph, s.x, s.y, s.z, v.x, v.y, v.z, s.rho, s.p, a.SP[j], a.SV[j], a.SW[j], ap, av, lv);
             cx += valid ? ap.x + av.x : 0.0f;
             cy += valid ? ap.y + av.y : 0.0f;
             cz += valid ? ap.z + av.z : 0.0f;
@@ -1009,9 +1284,10 @@ __device__ __forceinline__ void momentum_finish(const SphArgs& a, const PairSelf
     const double nvy = a.vy[i] + hdt * (double)ay;
     const double nvz = a.vz[i] + hdt * (double)az;
     a.ovx[i] = nvx; a.ovy[i] = nvy; a.ovz[i] = nvz;
-    const float4 nV = make_float4((float)nvx, (float)nvy, (float)nvz, s.w);
+    const float4 nV = make_float4((float)nvx, (float)nvy, (float)nvz, a.V[i].w);
     a.oV[i] = nV;
     if (FIRST) {
+        const FluidPos s = a.P[i];
         FluidPos o;
         o.x = s.x + a.dt * nvx;
         o.y = s.y + a.dt * nvy;
@@ -1019,7 +1295,7 @@ __device__ __forceinline__ void momentum_finish(const SphArgs& a, const PairSelf
         o.rho = s.rho;
         o.p = s.p;
         a.oP[i] = o;
-        if (a.GRout) st_grec(a.GRout, a.nf, i, grec(a.grid, a.pcell[i], o, nV));
+        if (a.GRout) st_grec(a.GRout, a.nf, i, a.fix, o, nV);
     }
 }
 
@@ -1045,14 +1321,13 @@ __device__ __forceinline__ void load_entries(const int* __restrict__ p, int* v)
 }
 
 template <int LANES, class LoadF, class UseF>
-__device__ __forceinline__ void for_entries(const int* __restrict__ list, int n, int nf, int i, int q, int safe,
+__device__ __forceinline__ void for_entries(const int* __restrict__ list, int n, int K, int i, int q, int safe,
                                             LoadF&& load, UseF&& use)
 {
     static_assert(LANES == 2 || LANES == 4 || LANES == 8, "entry-split pair loops take 2, 4 or 8 lanes");
     constexpr int E = kChunk / LANES;
     constexpr int CB = E >= kBatch ? 1 : kBatch / E;  // chunks per batch
-    const int* L = list + (size_t)i * kChunk + q * E;
-    const size_t cs = (size_t)nf * kChunk;
+    const int* L = list + list_entry(i, 0, K) + q * E;
     const int nch = (n + kChunk - 1) / kChunk;
     for (int c0 = 0; c0 < nch; c0 += CB) {
         int js[CB * E];
@@ -1061,7 +1336,7 @@ __device__ __forceinline__ void for_entries(const int* __restrict__ list, int n,
             const int c = c0 + cb;
             int v[E];
             if (c < nch) {
-                load_entries<E>(L + (size_t)c * cs, v);
+                load_entries<E>(L + c * kListStride, v);
             } else {
 #pragma unroll
                 for (int e = 0; e < E; e++) v[e] = safe;
@@ -1081,18 +1356,17 @@ __device__ __forceinline__ void for_entries(const int* __restrict__ list, int n,
 // list capacity, loaded in one go whatever the particle's count.
 constexpr int kPreEntries = 16;
 template <int LANES>
-__device__ __forceinline__ void preload_entries(const int* __restrict__ list, int K, int nf, int i, int q,
+__device__ __forceinline__ void preload_entries(const int* __restrict__ list, int K, int i, int q,
                                                 int (&pre)[kPreEntries])
 {
     constexpr int E = kChunk / LANES;
     constexpr int PC = kPreEntries / E;
     const int kch = K / kChunk;  // chunks of capacity (uniform)
-    const int* L = list + (size_t)i * kChunk + q * E;
-    const size_t cs = (size_t)nf * kChunk;
+    const int* L = list + list_entry(i, 0, K) + q * E;
 #pragma unroll
     for (int c = 0; c < PC; c++) {
         if (c < kch) {
-            load_entries<E>(L + (size_t)c * cs, &pre[c * E]);
+            load_entries<E>(L + c * kListStride, &pre[c * E]);
         } else {
 #pragma unroll
             for (int e = 0; e < E; e++) pre[c * E + e] = 0;
@@ -1104,7 +1378,7 @@ __device__ __forceinline__ void preload_entries(const int* __restrict__ list, in
 // preload_entries.  Same entries, same order.
 template <int LANES, class LoadF, class UseF>
 __device__ __forceinline__ void for_entries_pre(const int (&pre)[kPreEntries], const int* __restrict__ list, int n,
-                                                int nf, int i, int q, int safe, LoadF&& load, UseF&& use)
+                                                int K, int i, int q, int safe, LoadF&& load, UseF&& use)
 {
     constexpr int E = kChunk / LANES;
     constexpr int CB = E >= kBatch ? 1 : kBatch / E;  // chunks per batch
@@ -1126,15 +1400,14 @@ __device__ __forceinline__ void for_entries_pre(const int (&pre)[kPreEntries], c
         for (int k = 0; k < CB * E; k++) use(rec[k], js[k], (c0 + k / E) * kChunk + q * E + k % E < n);
     }
     if (nch <= PC) return;
-    const int* L = list + (size_t)i * kChunk + q * E;
-    const size_t cs = (size_t)nf * kChunk;
+    const int* L = list + list_entry(i, 0, K) + q * E;
     for (int c0 = PC; c0 < nch; c0 += CB) {
         int js[CB * E];
 #pragma unroll
         for (int cb = 0; cb < CB; cb++) {
             const int c = c0 + cb;
             int v[E];
-            load_entries<E>(L + (size_t)min(c, nch - 1) * cs, v);
+            load_entries<E>(L + min(c, nch - 1) * kListStride, v);
 #pragma unroll
             for (int e = 0; e < E; e++) js[cb * E + e] = c * kChunk + q * E + e < n ? v[e] : safe;
         }
@@ -1146,40 +1419,81 @@ __device__ __forceinline__ void for_entries_pre(const int (&pre)[kPreEntries], c
     }
 }
 
+// A particle with a far pair: its lists on the FP64 records, lane q taking
+// entries q, q + LANES, ...
+template <int LANES>
+__device__ __forceinline__ void momentum_far(const SphArgs& a, int i, int q, int nf, int nd, float& ax, float& ay,
+                                             float& az)
+{
+    const PairSelf s = pair_self<true>(a, i);
+#pragma unroll 1
+    for (int k = q; k < nf; k += LANES) {
+        const int j = a.nbr_ff[list_entry(i, k, a.K_ff)];
+        momentum_ff<true>(a, s, FluidRec{a.P[j], a.V[j]}, true, ax, ay, az);
+    }
+#pragma unroll 1
+    for (int k = q; k < nd; k += LANES) {
+        const int j = a.nbr_fd[list_entry(i, k, a.K_fd)];
+        momentum_fd<true>(a, s, DummyRec{a.DP[j], a.DV[j]}, j, true, ax, ay, az);
+    }
+}
+
 // updateWCSPHAccelerationKernel (WCSPHIntegrationKernel.cu:42-148) fused
 // with the half kick (:150-159) and, in the first half, the drift (:161-170).
-template <bool FIRST, bool UNIF, int LANES, bool GR = false>
+template <bool FIRST, bool UNIF, int LANES, bool GR, bool BALLS>
 __global__ __launch_bounds__(kThreads) void k_momentum(SphArgs a)
 {
-    const int g = xcd_block() * kThreads + threadIdx.x;
+    const int g = xcd_block_spread<32>() * kThreads + threadIdx.x;
     const int i = g / LANES, q = g % LANES;
     if (i >= a.nf) return;  // uniform over a lane group
-    const PairSelf s = pair_self<UNIF>(a, i);
     float ax = 0.f, ay = 0.f, az = 0.f;
     const auto load_f = [&](int j) { return FluidRec{ld_at(a.P, j), ld_at(a.V, j)}; };
     const auto load_d = [&](int j) { return DummyRec{ld_at(a.DP, j), ld_at(a.DV, j)}; };
-    const auto use_f = [&](const FluidRec& R, int, bool valid) { momentum_ff<UNIF>(a, s, R, valid, ax, ay, az); };
-    const auto use_d = [&](const DummyRec& R, int j, bool valid) { momentum_fd<UNIF>(a, s, R, j, valid, ax, ay, az); };
     if constexpr (GR) {
         static_assert(UNIF && LANES >= 2, "gather records: uniform scenes, entry-split lanes");
-        int pre[kPreEntries];
-        preload_entries<LANES>(a.nbr_ff, a.K_ff, a.nf, i, q, pre);
-        for_entries_pre<LANES>(pre, a.nbr_ff, min(a.cnt_ff[i], a.K_ff), a.nf, i, q, i,
-                               [&](int e) { return ld_grec(a.GRin, a.nf, e & kSlotMask); },
-                               [&](const GRec& R, int e, bool valid) {
-                                   momentum_ff_g(a, s, R, e >> kCodeShift, valid, ax, ay, az);
-                               });
-        if (a.nd > 0) for_entries<LANES>(a.nbr_fd, min(a.cnt_fd[i], a.K_fd), a.nf, i, q, 0, load_d, use_d);
-    } else if constexpr (LANES >= 2) {
-        int pre[kPreEntries];
-        preload_entries<LANES>(a.nbr_ff, a.K_ff, a.nf, i, q, pre);
-        for_entries_pre<LANES>(pre, a.nbr_ff, min(a.cnt_ff[i], a.K_ff), a.nf, i, q, i, load_f, use_f);
-        if (a.nd > 0) for_entries<LANES>(a.nbr_fd, min(a.cnt_fd[i], a.K_fd), a.nf, i, q, 0, load_d, use_d);
+        const int cf = a.cnt_ff[i], cd = a.nd > 0 ? a.cnt_fd[i] : 0;
+        const int nf = min(list_count(cf), a.K_ff), nd = min(list_count(cd), a.K_fd);
+        if ((cf | cd) & kFarBit) {
+            momentum_far<LANES>(a, i, q, nf, nd, ax, ay, az);
+        } else {
+            int pre[kPreEntries];
+            preload_entries<LANES>(a.nbr_ff, a.K_ff, i, q, pre);
+            const PairSelf s = pair_self_rec(a, i);
+            const float half_invh_u = a.ff_half_invh, half_c = 0.5f * s.ph.c;
+            MomentumSums m{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            for_entries_pre<LANES>(pre, a.nbr_ff, nf, a.K_ff, i, q, i, [&](int j) { return ld_grec(a.GRin, a.nf, j); },
+                                   [&](const GRec& R, int, bool) { momentum_ff_g(s, R, half_invh_u, half_c, m); });
+            const float k = a.ff_coef * s.inv_rho, kv = 2.0f * s.ph.nu * k;
+            ax = kv * m.vx - k * m.px;
+            ay = kv * m.vy - k * m.py;
+            az = kv * m.vz - k * m.pz;
+            if (nd > 0) {
+                MomentumSums w{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                for_entries<LANES>(a.nbr_fd, nd, a.K_fd, i, q, 0,
+                                   [&](int j) { return DummyFix{ld_at(a.DA, j), ld_at(a.DB, j), ld_at(a.DC, j)}; },
+                                   [&](const DummyFix& R, int, bool valid) { momentum_fd_g(a, s, R, valid, w); });
+                const float kd = a.fd_coef * s.inv_rho, kvd = (s.ph.nu + a.phd.nu) * kd;
+                ax += kvd * w.vx - kd * w.px;
+                ay += kvd * w.vy - kd * w.py;
+                az += kvd * w.vz - kd * w.pz;
+            }
+        }
     } else {
-        for_chunks_gathered<LANES>(a.nbr_ff, a.cnt_ff[i], a.K_ff, a.nf, i, q, i, load_f, use_f);
-        if (a.nd > 0) for_chunks_gathered<LANES>(a.nbr_fd, a.cnt_fd[i], a.K_fd, a.nf, i, q, 0, load_d, use_d);
+        const PairSelf s = pair_self<UNIF>(a, i);
+        const auto use_f = [&](const FluidRec& R, int, bool valid) { momentum_ff<UNIF>(a, s, R, valid, ax, ay, az); };
+        const auto use_d = [&](const DummyRec& R, int j, bool valid) { momentum_fd<UNIF>(a, s, R, j, valid, ax, ay, az); };
+        if constexpr (LANES >= 2) {
+            int pre[kPreEntries];
+            preload_entries<LANES>(a.nbr_ff, a.K_ff, i, q, pre);
+            for_entries_pre<LANES>(pre, a.nbr_ff, min(list_count(a.cnt_ff[i]), a.K_ff), a.K_ff, i, q, i, load_f, use_f);
+            if (a.nd > 0)
+                for_entries<LANES>(a.nbr_fd, min(list_count(a.cnt_fd[i]), a.K_fd), a.K_fd, i, q, 0, load_d, use_d);
+        } else {
+            for_row(a.nbr_ff, a.cnt_ff[i], a.K_ff, i, i, load_f, use_f);
+            if (a.nd > 0) for_row(a.nbr_fd, a.cnt_fd[i], a.K_fd, i, 0, load_d, use_d);
+        }
     }
-    momentum_finish<FIRST, LANES>(a, s, i, q, ax, ay, az);
+    momentum_finish<FIRST, LANES, BALLS>(a, i, q, ax, ay, az);
 }
 
 // One fluid neighbour's term of updateWCSPHDensityChangeKernel
@@ -1227,58 +1541,102 @@ __device__ __forceinline__ float continuity_fd(const SphArgs& a, const PairSelf&
 }
 
 // Coupled balls, lane-group sum and the EOS update (:266-282).
-template <int LANES>
-__device__ __forceinline__ void continuity_finish(const SphArgs& a, const PairSelf& s, int i, int q, float d)
+template <int LANES, bool BALLS>
+__device__ __forceinline__ void continuity_finish(const SphArgs& a, const Phase& ph, int i, int q, float d)
 {
-    if (a.ns > 0) {
+    if constexpr (BALLS) {
+        const FluidPos s = a.P[i];
+        const float4 v = a.V[i];
         for_chunks<LANES>(a.nbr_fs, a.cnt_fs[i], a.K_fs, a.nf, i, q, 0, [&](int j, bool valid) {
-            const float t = fs_density(a, s.ph, s.x, s.y, s.z, s.vx, s.vy, s.vz, s.rho, s.p, a.SP[j], a.SV[j], a.SW[j]);
+            const float t = fs_density(a, ph, s.x, s.y, s.z, v.x, v.y, v.z, s.rho, s.p, a.SP[j], a.SV[j], a.SW[j]);
             d += valid ? t : 0.0f;
         });
     }
     if (LANES > 1) d = lane_group_sum<LANES>(d);
     if (q != 0) return;
+    const FluidPos s = a.P[i];
     const float nd = a.drho[i] + (float)(a.dt * (double)(2.0f * s.rho * d));
     a.odrho[i] = nd;
     FluidPos o;
     o.x = s.x; o.y = s.y; o.z = s.z;
-    eos_eval(a.eos, a.gamma, s.ph, nd, o.rho, o.p);
+    eos_eval(a.eos, a.gamma, ph, nd, o.rho, o.p);
     a.oP[i] = o;
-    if (a.GRout) st_grec(a.GRout, a.nf, i, grec(a.grid, a.pcell[i], o, make_float4(s.vx, s.vy, s.vz, s.w)));
+    if (a.GRout) {
+        const float4 h = a.GRin[i], v = a.GRin[a.nf + i];
+        a.GRout[i] = make_float4(h.x, h.y, h.z, o.rho);
+        a.GRout[a.nf + i] = make_float4(o.p, v.y, v.z, v.w);
+    }
+}
+
+// continuity_ff and continuity_fd of a particle with a far pair.
+template <int LANES>
+__device__ __forceinline__ float continuity_far(const SphArgs& a, int i, int q, int nf, int nd)
+{
+    const PairSelf s = pair_self<true>(a, i);
+    float d = 0.f;
+#pragma unroll 1
+    for (int k = q; k < nf; k += LANES) {
+        const int j = a.nbr_ff[list_entry(i, k, a.K_ff)];
+        d += continuity_ff<true>(a, s, FluidRec{a.P[j], a.V[j]}, true);
+    }
+#pragma unroll 1
+    for (int k = q; k < nd; k += LANES) {
+        const int j = a.nbr_fd[list_entry(i, k, a.K_fd)];
+        d += continuity_fd<true>(a, s, DummyRec{a.DP[j], a.DV[j]}, j, true);
+    }
+    return d;
 }
 
 // updateWCSPHDensityChangeKernel (WCSPHIntegrationKernel.cu:172-264) fused
 // with the EOS update (:266-282).
-template <bool UNIF, int LANES, bool GR = false>
+template <bool UNIF, int LANES, bool GR, bool BALLS>
 __global__ __launch_bounds__(kThreads) void k_continuity(SphArgs a)
 {
-    const int g = xcd_block() * kThreads + threadIdx.x;
+    const int g = xcd_block_spread<32>() * kThreads + threadIdx.x;
     const int i = g / LANES, q = g % LANES;
     if (i >= a.nf) return;  // uniform over a lane group
-    const PairSelf s = pair_self<UNIF>(a, i);
     float d = 0.f;
     const auto load_f = [&](int j) { return FluidRec{ld_at(a.P, j), ld_at(a.V, j)}; };
     const auto load_d = [&](int j) { return DummyRec{ld_at(a.DP, j), ld_at(a.DV, j)}; };
-    const auto use_f = [&](const FluidRec& R, int, bool valid) { d += continuity_ff<UNIF>(a, s, R, valid); };
-    const auto use_d = [&](const DummyRec& R, int j, bool valid) { d += continuity_fd<UNIF>(a, s, R, j, valid); };
     if constexpr (GR) {
         static_assert(UNIF && LANES >= 2, "gather records: uniform scenes, entry-split lanes");
-        int pre[kPreEntries];
-        preload_entries<LANES>(a.nbr_ff, a.K_ff, a.nf, i, q, pre);
-        for_entries_pre<LANES>(pre, a.nbr_ff, min(a.cnt_ff[i], a.K_ff), a.nf, i, q, i,
-                               [&](int e) { return ld_grec(a.GRin, a.nf, e & kSlotMask); },
-                               [&](const GRec& R, int e, bool valid) { d += continuity_ff_g(a, s, R, e >> kCodeShift, valid); });
-        if (a.nd > 0) for_entries<LANES>(a.nbr_fd, min(a.cnt_fd[i], a.K_fd), a.nf, i, q, 0, load_d, use_d);
-    } else if constexpr (LANES >= 2) {
-        int pre[kPreEntries];
-        preload_entries<LANES>(a.nbr_ff, a.K_ff, a.nf, i, q, pre);
-        for_entries_pre<LANES>(pre, a.nbr_ff, min(a.cnt_ff[i], a.K_ff), a.nf, i, q, i, load_f, use_f);
-        if (a.nd > 0) for_entries<LANES>(a.nbr_fd, min(a.cnt_fd[i], a.K_fd), a.nf, i, q, 0, load_d, use_d);
+        const int cf = a.cnt_ff[i], cd = a.nd > 0 ? a.cnt_fd[i] : 0;
+        const int nf = min(list_count(cf), a.K_ff), nd = min(list_count(cd), a.K_fd);
+        if ((cf | cd) & kFarBit) {
+            d = continuity_far<LANES>(a, i, q, nf, nd);
+        } else {
+            int pre[kPreEntries];
+            preload_entries<LANES>(a.nbr_ff, a.K_ff, i, q, pre);
+            const PairSelf s = pair_self_rec(a, i);
+            const float half_invh_u = a.ff_half_invh, half_c = 0.5f * s.ph.c, rho_c = s.rho * half_c;
+            for_entries_pre<LANES>(pre, a.nbr_ff, nf, a.K_ff, i, q, i, [&](int j) { return ld_grec(a.GRin, a.nf, j); },
+                                   [&](const GRec& R, int, bool) { continuity_ff_g(s, R, half_invh_u, half_c, rho_c, d); });
+            d *= 0.5f * a.ff_coef;
+            if (nd > 0) {
+                float w = 0.f;
+                for_entries<LANES>(a.nbr_fd, nd, a.K_fd, i, q, 0,
+                                   [&](int j) { return DummyFix{ld_at(a.DA, j), ld_at(a.DB, j), ld_at(a.DC, j)}; },
+                                   [&](const DummyFix& R, int, bool valid) { continuity_fd_g(a, s, R, valid, w); });
+                d += 0.5f * a.fd_coef * w;
+            }
+        }
+        continuity_finish<LANES, BALLS>(a, a.phf, i, q, d);
     } else {
-        for_chunks_gathered<LANES>(a.nbr_ff, a.cnt_ff[i], a.K_ff, a.nf, i, q, i, load_f, use_f);
-        if (a.nd > 0) for_chunks_gathered<LANES>(a.nbr_fd, a.cnt_fd[i], a.K_fd, a.nf, i, q, 0, load_d, use_d);
+        const PairSelf s = pair_self<UNIF>(a, i);
+        const auto use_f = [&](const FluidRec& R, int, bool valid) { d += continuity_ff<UNIF>(a, s, R, valid); };
+        const auto use_d = [&](const DummyRec& R, int j, bool valid) { d += continuity_fd<UNIF>(a, s, R, j, valid); };
+        if constexpr (LANES >= 2) {
+            int pre[kPreEntries];
+            preload_entries<LANES>(a.nbr_ff, a.K_ff, i, q, pre);
+            for_entries_pre<LANES>(pre, a.nbr_ff, min(list_count(a.cnt_ff[i]), a.K_ff), a.K_ff, i, q, i, load_f, use_f);
+            if (a.nd > 0)
+                for_entries<LANES>(a.nbr_fd, min(list_count(a.cnt_fd[i]), a.K_fd), a.K_fd, i, q, 0, load_d, use_d);
+        } else {
+            for_row(a.nbr_ff, a.cnt_ff[i], a.K_ff, i, i, load_f, use_f);
+            if (a.nd > 0) for_row(a.nbr_fd, a.cnt_fd[i], a.K_fd, i, 0, load_d, use_d);
+        }
+        continuity_finish<LANES, BALLS>(a, s.ph, i, q, d);
     }
-    continuity_finish<LANES>(a, s, i, q, d);
 }
 
 // ----------------------------------------------------------- coupled balls
@@ -1351,11 +1709,11 @@ struct RevArgs {
     int* rfluid;
     int rcap;  // entries rfluid holds; a list overflow (reported by the fluid side) may exceed it
     double hf; // the fluid's smoothing length when it has one phase
-    // FP32 prefilter of the fluid positions (null: every test in FP64), as
-    // in the list walks: decisions outside the band are exact
-    const float4* Pf;
-    float band;
-    double R;
+    // fixed-point positions of the fluid (uniform scenes): candidates outside
+    // a band around the cut are decided by them, as in the list build
+    const float4* A;
+    FixGeom fix;
+    int prefilter;  // 0: every candidate takes the FP64 test
 };
 
 // Reverse index of the fluid -> ball lists: for ball j, the fluid slots i
@@ -1375,9 +1733,10 @@ __global__ __launch_bounds__(256) void k_fs_rev_walk(RevArgs a)
     const double bx = a.SP[j].x, by = a.SP[j].y, bz = a.SP[j].z;
     const Stencil st = make_stencil(g, bx, by, bz);
     int off = COUNT ? 0 : a.rstart[j];
-    const float4 bf = pos_f32(g, a.R, bx, by, bz);
-    const float c2 = (float)(4.0 * a.hf * a.hf);
-    const float band2 = bf.w != 0.f ? INFINITY : a.band * c2;
+    const Fix3 bq = fix_pos(a.fix, bx, by, bz);
+    float lo, hi;
+    // differences of up to 27 cells in FP32: 64 units a coordinate
+    cut_band(2.0 * a.hf * a.fix.inv, a.prefilter && !bq.far, 256.0f, 0.0f, lo, hi);
     for (int k = 0; k < 9; k++) {
         const int dz = k / 3 - 1, dy = k % 3 - 1;
         if (dz < st.loz || dz > st.hiz || dy < st.loy || dy > st.hiy) continue;
@@ -1394,13 +1753,14 @@ __global__ __launch_bounds__(256) void k_fs_rev_walk(RevArgs a)
         for (int base = s; base < e; base += 64) {
             const int i = base + lane;
             bool hit = false;
-            if (UNIF && a.Pf) {
+            if (UNIF) {
                 if (i < e) {
-                    const float4 q = a.Pf[i];
-                    const float fx = q.x - bf.x, fy = q.y - bf.y, fz = q.z - bf.z;
+                    const float4 q = a.A[i];
+                    const float fx = (float)(__float_as_int(q.x) - bq.x), fy = (float)(__float_as_int(q.y) - bq.y),
+                                fz = (float)(__float_as_int(q.z) - bq.z);
                     const float d2 = fx * fx + fy * fy + fz * fz;
-                    hit = d2 < c2;
-                    if ((q.w != 0.f) | (fabsf(d2 - c2) <= band2)) {
+                    hit = d2 < lo;
+                    if (!(q.w > 0.f) || (d2 < hi && !hit)) {
                         const FluidPos p = a.P[i];
                         hit = within_cut(2.0 * a.hf, p.x - bx, p.y - by, p.z - bz);
                     }
@@ -1589,9 +1949,8 @@ struct DummyReorderArgs {
     uint8_t* ophase;
     int* orig;
     int2* cells;
-    float4* DPf;  // FP32 positions for the list prefilter (null: none)
-    GridGeom grid;
-    double R;
+    float4* DA;  // fixed-point position (w: 1, or fix_mark's) for the list build
+    FixGeom fix;
 };
 
 __global__ __launch_bounds__(kThreads) void k_dummy_reorder(DummyReorderArgs a)
@@ -1604,7 +1963,8 @@ __global__ __launch_bounds__(kThreads) void k_dummy_reorder(DummyReorderArgs a)
     d.x = a.px[o]; d.y = a.py[o]; d.z = a.pz[o];
     d.nx = 0.f; d.ny = 0.f;
     a.DP[k] = d;
-    if (a.DPf) a.DPf[k] = pos_f32(a.grid, a.R, d.x, d.y, d.z);
+    const Fix3 q = fix_pos(a.fix, d.x, d.y, d.z);
+    a.DA[k] = fix_half(q, fix_mark(q, 1.0f));
     a.DV[k] = make_float4((float)a.vx[o], (float)a.vy[o], (float)a.vz[o], 0.f);
     a.ophase[k] = a.phase[o];
     const uint32_t h = a.skey[k];
@@ -1630,6 +1990,19 @@ __global__ void k_dummy_near(GridGeom g, long long numGrids, const int2* __restr
                 if (dcells[((long long)z * g.ny + y) * g.nx + x].x != -1) any = 1;
             }
     near[c] = any;
+}
+
+// The rest of the dummies' records, once their normals are known.
+__global__ __launch_bounds__(kThreads) void k_dummy_records(int n, const DummyPos* __restrict__ DP,
+                                                            const float4* __restrict__ DV, float4* __restrict__ DB,
+                                                            float2* __restrict__ DC)
+{
+    const int k = blockIdx.x * kThreads + threadIdx.x;
+    if (k >= n) return;
+    const DummyPos d = DP[k];
+    const float4 v = DV[k];
+    DB[k] = make_float4(d.nx, d.ny, v.w, v.x);
+    DC[k] = make_float2(v.y, v.z);
 }
 
 __global__ void k_dummy_hash(int n, GridGeom g, const double* __restrict__ px, const double* __restrict__ py,
@@ -1755,14 +2128,14 @@ struct demsph_sph {
     int* maxcount = nullptr;      // device [2]
     int* maxcount_h = nullptr;    // pinned [2]
     bool lists_valid = false;
-    // 32-byte gather records for the pair passes (uniform scenes): knob,
-    // whether the current lists carry cell codes, the two record buffers,
-    // each particle's packed cell at the last sort and stencil centre
+    // 32-byte gather records (uniform scenes): knob, state, the two buffers
+    // the passes of a step alternate between
     bool pair_records = true;
-    bool lists_coded = false;
+    bool rec_ready = false;  // GR[cG] holds the records of the current state
+    int cG = 0;
     GRec* GR[2] = {};  // nf records each, stored as split halves
     float4* gr(int b) const { return reinterpret_cast<float4*>(GR[b]); }
-    int *pcell = nullptr, *pcen = nullptr;
+    FixGeom fix{};
     // dummies
     DummyPos* DP = nullptr;
     float4* DV = nullptr;
@@ -1803,11 +2176,9 @@ struct demsph_sph {
     StepStamps stamps;  // step-end timestamps (batched serving)
     int pair_lanes_set = 0;  // 0: chosen from the particle count
     int list_lanes_set = 0;
-    // FP32 prefilter of the list walks (exact decisions; see pos_f32)
-    bool prefilter = true;
-    static constexpr float kPrefilterBand = 1.0e-3f;
-    double pref_R = 0.0;
-    float4 *Pf = nullptr, *DPf = nullptr;
+    bool prefilter = true;  // list candidates outside the cut's band are decided in fixed point
+    float4 *DA = nullptr, *DB = nullptr;  // dummy records (SphArgs)
+    float2* DC = nullptr;
 
     std::vector<demsph_couple*> couples;  // couplings holding this scene
 
@@ -1830,8 +2201,8 @@ struct demsph_sph {
         dfree(rank); dfree(key); dfree(skey); dfree(ktmp); dfree(perm); dfree(vtmp);
         dev_free(sort_temp);
         sort_temp = nullptr;
-        dfree(cells); dfree(nbr_ff); dfree(cnt_ff); dfree(nbr_fd); dfree(cnt_fd); dfree(Pf); dfree(DPf);
-        dfree(GR[0]); dfree(GR[1]); dfree(pcell); dfree(pcen);
+        dfree(cells); dfree(nbr_ff); dfree(cnt_ff); dfree(nbr_fd); dfree(cnt_fd); dfree(DA); dfree(DB); dfree(DC);
+        dfree(GR[0]); dfree(GR[1]);
         dfree(maxcount);
         host_free(maxcount_h);
         maxcount_h = nullptr;
@@ -1874,8 +2245,14 @@ struct demsph_sph {
         a.odrho = drho[1 - cD];
         a.nbr_ff = nbr_ff; a.cnt_ff = cnt_ff; a.nbr_fd = nbr_fd; a.cnt_fd = cnt_fd;
         a.K_ff = K_ff; a.K_fd = K_fd;
-        a.pcell = pcell; a.pcen = pcen; a.grid = grid;
-        a.DP = DP; a.DV = DV; a.dphase = dphase;
+        a.fix = fix;
+        const GradK gk = grad_k(phf.hf);
+        a.ff_half_invh = (float)(gk.half_invh / fix.inv);
+        a.ff_coef = (float)((double)gk.coef * phf.m / fix.inv);
+        const GradK gd = grad_k(0.5f * (phf.hf + phd.hf));
+        a.fd_half_invh = (float)(gd.half_invh / fix.inv);
+        a.fd_coef = (float)((double)gd.coef * phd.m / fix.inv);
+        a.DP = DP; a.DV = DV; a.dphase = dphase; a.DA = DA; a.DB = DB; a.DC = DC;
         a.ns = solids.ns; a.SP = solids.SP; a.SV = solids.SV; a.SW = solids.SW;
         a.nbr_fs = solids.nbr_fs; a.cnt_fs = solids.cnt_fs; a.K_fs = solids.K_fs; a.acs = solids.acs;
         a.gx = (float)g[0]; a.gy = (float)g[1]; a.gz = (float)g[2];
@@ -1897,8 +2274,8 @@ struct demsph_sph {
         if ((long long)std::max(K_ff, K_fd) * std::max(nf, 1) >= (1ll << 31))
             throw CapacityError("neighbour lists of " + std::to_string(std::max(K_ff, K_fd)) + " entries for " +
                                 std::to_string(nf) + " fluid particles exceed 2^31 entries");
-        nbr_ff = dmalloc<int>((size_t)K_ff * (nf > 0 ? nf : 1));
-        nbr_fd = dmalloc<int>((size_t)K_fd * (nf > 0 ? nf : 1));
+        nbr_ff = dmalloc<int>(list_alloc(nf, K_ff));
+        nbr_fd = dmalloc<int>(list_alloc(nf, K_fd));
         lists_valid = false;
     }
 
@@ -1925,12 +2302,11 @@ struct demsph_sph {
         const size_t cells = grid_set(gg, minb, maxb, staged_cell_size()) ? (size_t)gg.numGrids() : 0;
         const size_t rec = sizeof(FluidPos) + sizeof(float4) + 3 * sizeof(double) + sizeof(float) + sizeof(int);
         const size_t per_fluid = 2 * rec + rec + sizeof(int)             // two buffers, checkpoint, rank
-                                 + sizeof(float4)                         // FP32 list-prefilter copy
-                                 + 2 * sizeof(GRec) + 2 * sizeof(int)     // gather records, cells
+                                 + 2 * sizeof(GRec)                       // gather records
                                  + 2 * sizeof(int)                        // list counts
                                  + sizeof(int) * (size_t)(round_chunk(K_ff) + round_chunk(K_fd));
         const size_t per_sort = 3 * sizeof(uint32_t) + 2 * sizeof(int);
-        const size_t per_dummy = sizeof(DummyPos) + 2 * sizeof(float4) + 1 + sizeof(int);
+        const size_t per_dummy = sizeof(DummyPos) + 3 * sizeof(float4) + sizeof(float2) + 1 + sizeof(int);
         // initialisation uploads positions, velocities and phases through
         // temporary buffers, which the runtime's allocator keeps cached
         const size_t upload = 6 * sizeof(double) + 1;
@@ -1987,20 +2363,21 @@ struct demsph_sph {
         perm = dmalloc<int>(nsort); vtmp = dmalloc<int>(nsort);
         DEMSPH_HIP(dev_malloc(&sort_temp, radix_sort_temp_bytes(nsort)));
         cells = dmalloc<int2>(numGrids);
-        Pf = dmalloc<float4>(nf);
-        DPf = dmalloc<float4>(nd > 0 ? nd : 1);
-        // Points within pref_R of the grid origin on every axis carry FP32
-        // copies whose rounding stays inside the prefilter band for pairs at
-        // the smallest cut: |d2_f32 - d2| <= 2 sqrt(3) cut 2^-22 R + O(2^-24)
-        // cut^2 <= band cut^2 / 2 for R = 500 cut_min.
+        const size_t md = nd > 0 ? nd : 1;
+        DA = dmalloc<float4>(md); DB = dmalloc<float4>(md); DC = dmalloc<float2>(md);
         {
-            double hmin = 1e300;
-            for (const Phase& q : phases) hmin = std::min(hmin, q.h);
-            pref_R = 500.0 * 2.0 * hmin;
+            fix.minx = grid.minx; fix.miny = grid.miny; fix.minz = grid.minz;
+            // a power of two of units to the fluid's 2 h makes the kernel
+            // argument r / 2h exact in the pair passes
+            const double cmax = std::max(grid.cx, std::max(grid.cy, grid.cz)), two_h = 1.0 / grad_k(phf.hf).half_invh;
+            fix.inv = two_h <= cmax && cmax <= 2.0 * two_h ? 0.5 * kFixPerCell / two_h : kFixPerCell / cmax;
+            fix.u = (float)(1.0 / fix.inv);
+            fix.ex = (grid.maxx - grid.minx) * fix.inv;
+            fix.ey = (grid.maxy - grid.miny) * fix.inv;
+            fix.ez = (grid.maxz - grid.minz) * fix.inv;
         }
         cnt_ff = dmalloc<int>(n); cnt_fd = dmalloc<int>(n);
         GR[0] = dmalloc<GRec>(n); GR[1] = dmalloc<GRec>(n);
-        pcell = dmalloc<int>(n); pcen = dmalloc<int>(n);
         maxcount = dmalloc<int>(3);
         DEMSPH_HIP(host_malloc((void**)&maxcount_h, 3 * sizeof(int)));
         alloc_lists();
@@ -2058,12 +2435,14 @@ struct demsph_sph {
             ra.px = ux; ra.py = uy; ra.pz = uz; ra.vx = wx; ra.vy = wy; ra.vz = wz; ra.phase = uph;
             ra.DP = DP; ra.DV = DV; ra.ophase = dphase;
             ra.orig = dorig; ra.cells = dcells;
-            ra.DPf = DPf; ra.grid = grid; ra.R = pref_R;
+            ra.DA = DA; ra.fix = fix;
             hipLaunchKernelGGL(k_dummy_reorder, dim3(blocks_for(m, kThreads)), dim3(kThreads), 0, stream, ra);
             NormalArgs na{};
             na.nd = (int)m; na.grid = grid; na.phases = d_phases; na.DP = DP; na.DV = DV;
             na.dphase = dphase; na.dcells = dcells;
             hipLaunchKernelGGL(k_dummy_normals, dim3(blocks_for(m, kThreads)), dim3(kThreads), 0, stream, na);
+            hipLaunchKernelGGL(k_dummy_records, dim3(blocks_for(m, kThreads)), dim3(kThreads), 0, stream, (int)m, DP,
+                               DV, DB, DC);
             DEMSPH_HIP(hipGetLastError());
             DEMSPH_HIP(hipStreamSynchronize(stream));
             dfree(ux); dfree(uy); dfree(uz); dfree(wx); dfree(wy); dfree(wz); dfree(uph);
@@ -2119,9 +2498,8 @@ struct demsph_sph {
         ra.oP = P[1 - cP]; ra.oV = V[1 - cV]; ra.ovx = vx[1 - cV]; ra.ovy = vy[1 - cV]; ra.ovz = vz[1 - cV];
         ra.odrho = drho[1 - cD];
         ra.cells = cells;
-        ra.oPf = prefilter ? Pf : nullptr; ra.grid = grid; ra.R = pref_R;
-        const bool coded = records_usable();
-        ra.oGR = coded ? gr(0) : nullptr; ra.opcell = pcell;
+        ra.fix = fix;
+        ra.oGR = gr(0); ra.rec_full = records_usable() ? 1 : 0;
         DEMSPH_LAUNCH(timer, "sph_reorder", k_reorder, gb, tb, 0, stream, ra);
         cP ^= 1; cV ^= 1; cD ^= 1; cO ^= 1;
         cells_track_skey = true;
@@ -2131,60 +2509,67 @@ struct demsph_sph {
         la.DP = DP; la.dphase = dphase; la.dcells = dcells; la.dummy_near = dummy_near;
         la.nbr_ff = nbr_ff; la.cnt_ff = cnt_ff; la.nbr_fd = nbr_fd; la.cnt_fd = cnt_fd;
         la.K_ff = K_ff; la.K_fd = K_fd; la.maxcount = maxcount;
-        la.Pf = Pf; la.DPf = DPf; la.band = kPrefilterBand;
-        la.pcen = coded ? pcen : nullptr;
-        lists_coded = coded;
+        la.A = gr(0); la.DA = DA; la.skey = skey; la.numGrids = numGrids;
+        const double edge = std::max(grid.cx, std::max(grid.cy, grid.cz)) * fix.inv;
+        la.reach = (float)(0.75 * edge);
+        la.err = list_error(la.reach, edge);
+        cut_band(2.0 * phf.h * fix.inv, prefilter, kListSlack, la.err, la.lo_f, la.hi_f);
+        cut_band(2.0 * std::max(phf.h, phd.h) * fix.inv, prefilter, kListSlack, la.err, la.lo_d, la.hi_d);
+        la.stepx = (unsigned long long)(grid.cx * fix.inv * 1048576.0 + 0.5);
+        la.stepy = (unsigned long long)(grid.cy * fix.inv * 1048576.0 + 0.5);
+        la.stepz = (unsigned long long)(grid.cz * fix.inv * 1048576.0 + 0.5);
+        la.inv = fix.inv; la.prefilter = prefilter ? 1 : 0;
+        cG = 0;
+        rec_ready = ra.rec_full != 0;
         if (uniform) lists_lanes<true>(la);
         else lists_lanes<false>(la);
         lists_valid = true;
     }
 
-    // Lanes per fluid particle in the list build: the fewest of 4, 8 that
-    // put 600k threads in flight (measured on MI355X: 8 lanes at 2.7k and
-    // 35k particles, 4 at 256k and 741k, where 4 beat 2 by 10 and 4 %).
+    // Lanes per fluid particle in the list build (a wave takes 64 / lanes
+    // particles): the fewest of 2, 4, 8 that put 600k threads in flight.
+    // More particles a wave share more of its candidate loads, and fewer
+    // waves hide less of each other's latencies.  Measured with 8 / 4 / 2
+    // lanes, us: 2k particles 26 / 34 / 54, 18k 29 / 38 / 61, 60k 53 / 54 /
+    // 79, 256k 133 / 117 / 128, 1M 429 / 340 / 314.
     int list_lanes() const
     {
         if (list_lanes_set > 0) return list_lanes_set;
         return list_lanes_rule();
     }
-    int list_lanes_rule() const { return lanes_for(600000, 4); }
+    int list_lanes_rule() const { return lanes_for(600000, 2); }
     int lanes_for(long long fill, int least = 2) const
     {
         int L = least;
         while (L < 8 && (long long)nf * L < fill) L *= 2;
         return L;
     }
-    template <bool U, int L>
-    void lists_launch(const ListArgs& la)
+    // Below these sizes a wave takes one kind of neighbour, or four slots: the
+    // chip has lanes to spare and the build lasts as long as its longest wave,
+    // 8 us to the first candidates, 1.2 us a set and 0.5 us per 64 candidates.
+    // One kind a wave, 2k / 18k / 60k / 120k particles: 27 -> 22, 32 -> 26
+    // (48 -> 32 with a spray of one set per particle), 55 -> 52, 77 -> 80 us;
+    // four slots as well: 22 -> 19, 26 -> 28 us.
+    static constexpr int kListOneKind = 80000, kListFour = 6000;
+    template <bool U, int G>
+    void lists_launch(const ListArgs& la, int per_wave)
     {
-        const dim3 gb(blocks_for((long long)nf * L, kThreads)), tb(kThreads);
-        if constexpr (U) {
-            if (la.pcen) {
-                if (L > 1 && prefilter)
-                    DEMSPH_LAUNCH(timer, "sph_lists", (k_build_lists<U, L, true, true>), gb, tb, 0, stream, la);
-                else DEMSPH_LAUNCH(timer, "sph_lists", (k_build_lists<U, L, false, true>), gb, tb, 0, stream, la);
-                return;
-            }
-        }
-        if (L > 1 && prefilter)
-            DEMSPH_LAUNCH(timer, "sph_lists", (k_build_lists<U, L, true, false>), gb, tb, 0, stream, la);
-        else DEMSPH_LAUNCH(timer, "sph_lists", (k_build_lists<U, L, false, false>), gb, tb, 0, stream, la);
+        const dim3 gb(blocks_for(blocks_for(nf, per_wave), kThreads / 64), nd > 0 && nf <= kListOneKind ? 2 : 1), tb(kThreads);
+        DEMSPH_LAUNCH(timer, "sph_lists", (k_build_lists<U, G>), gb, tb, 0, stream, la, per_wave);
     }
-    // Gather records and coded lists need one phase, slots below 2^25 and a
-    // grid of at most 2048 x 2048 x 1024 cells, and the entry-split passes.
-    bool records_usable() const
-    {
-        return pair_records && uniform && nf > 0 && nf <= kSlotMask && grid.nx <= 2048 && grid.ny <= 2048 &&
-               grid.nz <= 1024 && pair_lanes() >= 2;
-    }
+    // The pair passes of uniform scenes gather records unless one lane keeps
+    // the sums in list order.
+    bool records_usable() const { return pair_records && uniform && nf > 0 && pair_lanes() >= 2; }
     template <bool U>
     void lists_lanes(const ListArgs& la)
     {
         switch (list_lanes()) {
-        case 2: lists_launch<U, 2>(la); break;
-        case 4: lists_launch<U, 4>(la); break;
-        case 8: lists_launch<U, 8>(la); break;
-        default: lists_launch<U, 1>(la); break;
+        case 8:
+            if (nf <= kListFour) lists_launch<U, 4>(la, 4);
+            else lists_launch<U, 8>(la, 8);
+            break;
+        case 4: lists_launch<U, 16>(la, 16); break;
+        default: lists_launch<U, 32>(la, 64 / list_lanes()); break;
         }
     }
 
@@ -2198,17 +2583,23 @@ struct demsph_sph {
         return lanes_for(400000, 4);
     }
 
-    template <bool FIRST, bool U, int L>
+    template <bool FIRST, bool U, int L, bool BALLS>
     void momentum_launch(const char* name, const SphArgs& a)
     {
         const dim3 gb(blocks_for((long long)nf * L, kThreads)), tb(kThreads);
         if constexpr (U && L >= 2) {
             if (a.GRin) {
-                DEMSPH_LAUNCH(timer, name, (k_momentum<FIRST, U, L, true>), gb, tb, 0, stream, a);
+                DEMSPH_LAUNCH(timer, name, (k_momentum<FIRST, U, L, true, BALLS>), gb, tb, 0, stream, a);
                 return;
             }
         }
-        DEMSPH_LAUNCH(timer, name, (k_momentum<FIRST, U, L>), gb, tb, 0, stream, a);
+        DEMSPH_LAUNCH(timer, name, (k_momentum<FIRST, U, L, false, BALLS>), gb, tb, 0, stream, a);
+    }
+    template <bool FIRST, bool U, int L>
+    void momentum_launch(const char* name, const SphArgs& a)
+    {
+        if (a.ns > 0) momentum_launch<FIRST, U, L, true>(name, a);
+        else momentum_launch<FIRST, U, L, false>(name, a);
     }
     template <bool FIRST, bool U>
     void momentum_lanes(const char* name, const SphArgs& a)
@@ -2220,17 +2611,23 @@ struct demsph_sph {
         default: momentum_launch<FIRST, U, 1>(name, a); break;
         }
     }
-    template <bool U, int L>
+    template <bool U, int L, bool BALLS>
     void continuity_launch(const SphArgs& a)
     {
         const dim3 gb(blocks_for((long long)nf * L, kThreads)), tb(kThreads);
         if constexpr (U && L >= 2) {
             if (a.GRin) {
-                DEMSPH_LAUNCH(timer, "sph_continuity", (k_continuity<U, L, true>), gb, tb, 0, stream, a);
+                DEMSPH_LAUNCH(timer, "sph_continuity", (k_continuity<U, L, true, BALLS>), gb, tb, 0, stream, a);
                 return;
             }
         }
-        DEMSPH_LAUNCH(timer, "sph_continuity", (k_continuity<U, L>), gb, tb, 0, stream, a);
+        DEMSPH_LAUNCH(timer, "sph_continuity", (k_continuity<U, L, false, BALLS>), gb, tb, 0, stream, a);
+    }
+    template <bool U, int L>
+    void continuity_launch(const SphArgs& a)
+    {
+        if (a.ns > 0) continuity_launch<U, L, true>(a);
+        else continuity_launch<U, L, false>(a);
     }
     template <bool U>
     void continuity_lanes(const SphArgs& a)
@@ -2243,11 +2640,31 @@ struct demsph_sph {
         }
     }
 
+    // Records for a pass: in use while every pass since the search wrote them.
+    void use_records(SphArgs& a, bool writes)
+    {
+        rec_ready = rec_ready && pair_lanes() >= 2;
+        if (!rec_ready) return;
+        a.GRin = gr(cG);
+        if (writes) {
+            a.GRout = gr(1 - cG);
+            cG ^= 1;
+        }
+    }
+    // After a host write to the state the records follow it.
+    void refresh_records()
+    {
+        if (!rec_ready) return;
+        hipLaunchKernelGGL(k_refresh_records, dim3(blocks_for(nf, kThreads)), dim3(kThreads), 0, stream, nf, fix, P[cP],
+                           V[cV], gr(cG));
+        DEMSPH_HIP(hipGetLastError());
+    }
+
     void first_half_enqueue(double dt)
     {
         SphArgs a = args();
         a.dt = dt;
-        if (lists_coded) { a.GRin = gr(0); a.GRout = gr(1); }
+        use_records(a, true);
         if (uniform) momentum_lanes<true, true>("sph_momentum_first", a);
         else momentum_lanes<true, false>("sph_momentum_first", a);
         cP ^= 1; cV ^= 1;
@@ -2257,7 +2674,7 @@ struct demsph_sph {
     {
         SphArgs a = args();
         a.dt = dt;
-        if (lists_coded) { a.GRin = gr(1); a.GRout = gr(0); }
+        use_records(a, true);
         if (uniform) continuity_lanes<true>(a);
         else continuity_lanes<false>(a);
         cP ^= 1; cD ^= 1;
@@ -2267,7 +2684,10 @@ struct demsph_sph {
     {
         SphArgs a = args();
         a.dt = dt;
-        if (lists_coded) a.GRin = gr(0);
+        use_records(a, false);
+        // the velocities change and the records do not: a further half
+        // before the next search takes the FP64 records
+        rec_ready = false;
         if (uniform) momentum_lanes<false, true>("sph_momentum_second", a);
         else momentum_lanes<false, false>("sph_momentum_second", a);
         cV ^= 1;
@@ -2845,10 +3265,11 @@ extern "C" int demsph_sph_get(demsph_sph* s, const char* field, void* out, size_
             if (!s->lists_valid) throw InvalidArg("no neighbour lists yet");
             const int K = ff ? s->K_ff : s->K_fd;
             auto cnt = fetch(ff ? s->cnt_ff : s->cnt_fd, n, st);
+            for (int& c : cnt) c = list_count(c);
             std::vector<int> byo(n);
             for (size_t i = 0; i < n; i++) byo[orig[i]] = cnt[i];
             if (f == "neighborCount" || f == "dummyNeighborCount") return emit(byo, out, capacity, count);
-            auto nbr = fetch(ff ? s->nbr_ff : s->nbr_fd, (size_t)K * n, st);
+            auto nbr = fetch(ff ? s->nbr_ff : s->nbr_fd, list_alloc((int)n, K), st);
             std::vector<int> rankh(n);
             for (size_t i = 0; i < n; i++) rankh[orig[i]] = (int)i;
             std::vector<int> dor;
@@ -2858,8 +3279,7 @@ extern "C" int demsph_sph_get(demsph_sph* s, const char* field, void* out, size_
                 const int i = rankh[o];
                 const int c = std::min(cnt[i], K);
                 for (int k = 0; k < c; k++) {
-                    int j = nbr[(((size_t)(k / kChunk) * n + i) * kChunk) + (k % kChunk)];
-                    if (ff && s->lists_coded) j &= kSlotMask;
+                    const int j = nbr[list_entry(i, k, K)];
                     v.push_back(ff ? orig[j] : dor[j]);
                 }
             }
@@ -3096,6 +3516,7 @@ extern "C" int demsph_sph_set(demsph_sph* s, const char* field, const void* in, 
             copy_sync(s->vy[b], hy.data(), n * 8, hipMemcpyHostToDevice, s->stream);
             copy_sync(s->vz[b], hz.data(), n * 8, hipMemcpyHostToDevice, s->stream);
             copy_sync(s->V[b], hv.data(), n * sizeof(float4), hipMemcpyHostToDevice, s->stream);
+            s->refresh_records();
             return;
         }
         if (f == "densityChange") {
@@ -3104,6 +3525,7 @@ extern "C" int demsph_sph_set(demsph_sph* s, const char* field, const void* in, 
             for (size_t i = 0; i < n; i++) h[i] = (float)src[orig[i]];
             copy_sync(s->drho[s->cD], h.data(), n * 4, hipMemcpyHostToDevice, s->stream);
             s->refresh_eos();
+            s->refresh_records();
             DEMSPH_HIP(hipStreamSynchronize(st));
             return;
         }
@@ -3410,10 +3832,9 @@ struct demsph_couple {
         ra.ns = ns; ra.grid = f->grid; ra.cells = f->cells; ra.P = f->P[f->cP]; ra.V = f->V[f->cV];
         ra.phases = f->d_phases; ra.SP = SP; ra.rcnt = rcnt; ra.rstart = rstart; ra.rfluid = rfluid; ra.rcap = rcap();
         ra.hf = f->phf.h;
-        // the fluid's FP32 copy is current when the search wrote it
-        ra.Pf = f->prefilter ? f->Pf : nullptr;
-        ra.band = demsph_sph::kPrefilterBand;
-        ra.R = f->pref_R;
+        ra.A = f->gr(0);  // as the search wrote it
+        ra.fix = f->fix;
+        ra.prefilter = f->prefilter ? 1 : 0;
         const dim3 wb(blocks_for(ns, kBallsPerBlock)), wt(64 * kBallsPerBlock);
         // one fluid phase: every fluid particle has the same support
         const bool unif = f->fluid_uniform();
