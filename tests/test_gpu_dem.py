@@ -165,6 +165,21 @@ def test_granular_collapse_matches_oracle():
     assert np.array_equal(g.get("triCancel"), o.get("tri_cancel"))
 
 
+def test_read_back_leaves_the_scene_alone():
+    """Reading between steps, before and after rebuilds of the pair lists (every
+    fifth step), returns positions in insertion order and changes nothing."""
+    s = random_scene()
+    a, b = ts.DEMSceneGPU(s), ts.DEMSceneGPU(s)
+    assert np.array_equal(a.get("position"), oracle.OracleDEM(s).get("pos"))
+    for k in range(12):
+        a.step(1)
+        b.step(1)
+        for f in ("position", "velocity", "angularVelocity", "force", "torque", "radius", "inverseMass"):
+            a.get(f)
+    for f in ("position", "velocity", "angularVelocity", "force", "torque", "slidingSpring", "objectPointing"):
+        assert np.array_equal(a.get(f), b.get(f)), f
+
+
 def test_clumps_on_plane_match_oracle():
     s = scenes.DEMScene("clumps")
     rng = np.random.default_rng(5)

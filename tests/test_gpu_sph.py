@@ -372,6 +372,35 @@ def test_records_follow_a_field_set_between_search_and_halves(field, small):
         assert np.abs(a - b).max() < 1e-5 * np.abs(b).max()
 
 
+@pytest.mark.parametrize("n", [1, 85, 256, 257])
+def test_read_back_in_insertion_order(n):
+    """Values come back in insertion order, unchanged, from sorted particles
+    (counts about the read-back kernel's blocks); a too small output is
+    refused; reading between the calls of a step leaves the step alone."""
+    import ctypes as C
+
+    rng = np.random.default_rng(n)
+    pos, vel = rng.uniform(0.0, 0.2, (n, 3)), rng.uniform(-1.0, 1.0, (n, 3))
+    spec = scenes.SPHSceneSpec(fluid_pos=pos, fluid_vel=vel, dummy_pos=np.zeros((0, 3)), dx=0.01, rho0=1000.0, c0=10.0,
+                               nu=1e-6, min_bound=np.zeros(3), max_bound=np.full(3, 0.2),
+                               gravity=np.array([0.0, 0.0, -9.81]), dt=1e-6)
+    a, b = make_gpu(spec), make_gpu(spec)
+    for s in (a, b):
+        s.neighbor_search()
+    assert np.array_equal(a.get("position"), pos) and np.array_equal(a.get("velocity"), vel)
+    assert a.get("density").shape == a.get("pressure").shape == a.get("densityChange").shape == (n,)
+    out, cnt = np.empty(3 * n), C.c_size_t()
+    for f in (b"position", b"velocity"):
+        assert ts.lib().demsph_sph_get(a._h, f, out.ctypes.data_as(C.c_void_p), 3 * n - 1, C.byref(cnt)) != 0
+    for s in (a, b):
+        s.first_half(spec.dt)
+    a.get("velocity")
+    for s in (a, b):
+        s.second_half(spec.dt)
+    for f in ("position", "velocity", "density", "densityChange"):
+        assert np.array_equal(a.get(f), b.get(f)), f
+
+
 def test_two_phases_match_oracle():
     """Two fluid phases of different spacing, density and viscosity side by
     side (the kernels' non-uniform paths: per-pair cuts, phase lookups,

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <array>
 #include <cstdint>
 #include <cstdio>
 #include <mutex>
@@ -308,5 +309,47 @@ struct StepStamps {
     int cap = 0;
 };
 void step_stamp(const StepStamps& st, hipStream_t s);
+
+// -------------------------------------------------------------- read-back
+// Values of sorted particles as doubles in insertion order, COMPS to a
+// particle; the output runs through the parts, n values each.
+template <class T, int COMPS>
+__global__ __launch_bounds__(256) void k_in_order(size_t n, std::array<const T*, 3> src, int stride,
+                                                  const int* __restrict__ orig, double* p0, double* p1, double* p2)
+{
+    const size_t k = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= n) return;
+    const size_t o = (size_t)orig[k];
+#pragma unroll
+    for (int c = 0; c < COMPS; c++) {
+        const size_t at = COMPS * o + c;
+        (at < n ? p0[at] : at < 2 * n ? p1[at - n] : p2[at - 2 * n]) = (double)src[c][k * stride];
+    }
+}
+// One kernel puts the values in order in scratch (parts of n doubles,
+// joined if they are one allocation, end to end) and the copies go straight to the caller's memory.  Copying the arrays and their
+// order to the host and scattering them there, on the query for the count as
+// well, was bound by the host.
+// Position and velocity of 2k / 18k / 256k / 1M particles: 0.33 -> 0.10,
+// 0.29 -> 0.10, 3.5 -> 0.74, 18.4 -> 2.7 ms; of 200k balls 2.3 -> 0.59 ms.
+template <class T, int COMPS>
+void read_in_order(size_t n, const std::array<const T*, 3>& src, int stride, const int* orig, double* const (&part)[3],
+                   bool joined, void* out, size_t capacity, size_t* count, hipStream_t st)
+{
+    if (count) *count = COMPS * n;
+    if (!out) return;
+    if (capacity < COMPS * n) throw InvalidArg("output capacity too small");
+    if (n) {
+        k_in_order<T, COMPS><<<dim3(blocks_for((long long)n, 256)), dim3(256), 0, st>>>(n, src, stride, orig, part[0],
+                                                                                       part[1], part[2]);
+        DEMSPH_HIP(hipGetLastError());
+        const int parts = joined ? 1 : COMPS;
+        const size_t m = COMPS * n / parts;
+        for (int c = 0; c < parts; c++)
+            DEMSPH_HIP(hipMemcpyAsync(static_cast<double*>(out) + c * m, part[c], m * sizeof(double),
+                                      hipMemcpyDeviceToHost, st));
+    }
+    DEMSPH_HIP(hipStreamSynchronize(st));
+}
 
 }  // namespace demsph

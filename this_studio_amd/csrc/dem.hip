@@ -3126,20 +3126,13 @@ extern "C" int demsph_dem_get(demsph_dem* d, const char* field, void* out, size_
         hipStream_t st = d->stream;
         const int cb = d->cb;
         const size_t n = d->n;
-        auto orig = fetch(d->borig[cb].p, n, st);
+        // the copies that the next sort fills are free between calls
+        double* const part[3] = {d->bpx[1 - cb].p, d->bpy[1 - cb].p, d->bpz[1 - cb].p};
         auto vec = [&](const DBuf<double>& x, const DBuf<double>& y, const DBuf<double>& z) {
-            auto hx = fetch(x.p, n, st), hy = fetch(y.p, n, st), hz = fetch(z.p, n, st);
-            std::vector<double> v(3 * n);
-            for (size_t i = 0; i < n; i++) {
-                v[3 * (size_t)orig[i]] = hx[i]; v[3 * (size_t)orig[i] + 1] = hy[i]; v[3 * (size_t)orig[i] + 2] = hz[i];
-            }
-            return v;
+            read_in_order<double, 3>(n, {x.p, y.p, z.p}, 1, d->borig[cb].p, part, false, out, capacity, count, st);
         };
         auto scal = [&](const DBuf<double>& x) {
-            auto hx = fetch(x.p, n, st);
-            std::vector<double> v(n);
-            for (size_t i = 0; i < n; i++) v[orig[i]] = hx[i];
-            return v;
+            read_in_order<double, 1>(n, {x.p}, 1, d->borig[cb].p, part, false, out, capacity, count, st);
         };
         auto plain3 = [&](const DBuf<double>& x, const DBuf<double>& y, const DBuf<double>& z, size_t m) {
             auto hx = fetch(x.p, m, st), hy = fetch(y.p, m, st), hz = fetch(z.p, m, st);
@@ -3154,13 +3147,14 @@ extern "C" int demsph_dem_get(demsph_dem* d, const char* field, void* out, size_
             for (size_t i = 0; i < m; i++) { v[4 * i] = ha[i]; v[4 * i + 1] = hb[i]; v[4 * i + 2] = hc[i]; v[4 * i + 3] = he[i]; }
             return v;
         };
-        if (f == "position") return emit(vec(d->bpx[cb], d->bpy[cb], d->bpz[cb]), out, capacity, count);
-        if (f == "velocity") return emit(vec(d->bvx[cb], d->bvy[cb], d->bvz[cb]), out, capacity, count);
-        if (f == "angularVelocity") return emit(vec(d->bwx[cb], d->bwy[cb], d->bwz[cb]), out, capacity, count);
-        if (f == "force") return emit(vec(d->fx, d->fy, d->fz), out, capacity, count);
-        if (f == "torque") return emit(vec(d->tx, d->ty, d->tz), out, capacity, count);
-        if (f == "radius") return emit(scal(d->br[cb]), out, capacity, count);
-        if (f == "inverseMass") return emit(scal(d->bim[cb]), out, capacity, count);
+        if (f == "position") return vec(d->bpx[cb], d->bpy[cb], d->bpz[cb]);
+        if (f == "velocity") return vec(d->bvx[cb], d->bvy[cb], d->bvz[cb]);
+        if (f == "angularVelocity") return vec(d->bwx[cb], d->bwy[cb], d->bwz[cb]);
+        if (f == "force") return vec(d->fx, d->fy, d->fz);
+        if (f == "torque") return vec(d->tx, d->ty, d->tz);
+        if (f == "radius") return scal(d->br[cb]);
+        if (f == "inverseMass") return scal(d->bim[cb]);
+        auto orig = fetch(d->borig[cb].p, n, st);
         if (f == "hashValue") {
             auto k = fetch(d->skey.p, n, st);
             return emit(std::vector<int>(k.begin(), k.end()), out, capacity, count);

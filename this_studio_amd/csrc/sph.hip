@@ -3206,36 +3206,22 @@ extern "C" int demsph_sph_get(demsph_sph* s, const char* field, void* out, size_
         const std::string f = field;
         hipStream_t st = s->stream;
         const size_t n = s->nf;
-        auto orig = fetch(s->orig[s->cO], n, st);
-        if (f == "position" || f == "density" || f == "pressure") {
-            auto h = fetch(s->P[s->cP], n, st);
-            const bool pos = f == "position";
-            std::vector<double> v(pos ? 3 * n : n);
-            for (size_t i = 0; i < n; i++) {
-                const size_t o = orig[i];
-                if (pos) {
-                    v[3 * o] = h[i].x; v[3 * o + 1] = h[i].y; v[3 * o + 2] = h[i].z;
-                } else {
-                    v[o] = f == "density" ? h[i].rho : h[i].p;
-                }
-            }
-            return emit(v, out, capacity, count);
-        }
-        if (f == "velocity") {
-            auto hx = fetch(s->vx[s->cV], n, st), hy = fetch(s->vy[s->cV], n, st), hz = fetch(s->vz[s->cV], n, st);
-            std::vector<double> v(3 * n);
-            for (size_t i = 0; i < n; i++) {
-                const size_t o = orig[i];
-                v[3 * o] = hx[i]; v[3 * o + 1] = hy[i]; v[3 * o + 2] = hz[i];
-            }
-            return emit(v, out, capacity, count);
-        }
-        if (f == "densityChange") {
-            auto h = fetch(s->drho[s->cD], n, st);
-            std::vector<double> v(n);
-            for (size_t i = 0; i < n; i++) v[orig[i]] = h[i];
-            return emit(v, out, capacity, count);
-        }
+        // the buffer that the next pass overwrites is free between calls
+        const int* const to = s->orig[s->cO];
+        const FluidPos* const P = s->P[s->cP];
+        double* const w = reinterpret_cast<double*>(s->P[1 - s->cP]);
+        static_assert(sizeof(FluidPos) == 4 * sizeof(double), "a record holds the three components");
+        double* const part[3] = {w, w + n, w + 2 * n};
+        if (f == "position")
+            return read_in_order<double, 3>(n, {&P->x, &P->y, &P->z}, 4, to, part, true, out, capacity, count, st);
+        if (f == "density") return read_in_order<float, 1>(n, {&P->rho}, 8, to, part, true, out, capacity, count, st);
+        if (f == "pressure") return read_in_order<float, 1>(n, {&P->p}, 8, to, part, true, out, capacity, count, st);
+        if (f == "velocity")
+            return read_in_order<double, 3>(n, {s->vx[s->cV], s->vy[s->cV], s->vz[s->cV]}, 1, to, part, true, out, capacity,
+                                            count, st);
+        if (f == "densityChange")
+            return read_in_order<float, 1>(n, {s->drho[s->cD]}, 1, to, part, true, out, capacity, count, st);
+        auto orig = fetch(to, n, st);
         if (f == "dummyNormal") {
             const size_t m = s->nd;
             auto dor = fetch(s->dorig, m, st);
