@@ -180,6 +180,24 @@ def test_read_back_leaves_the_scene_alone():
         assert np.array_equal(a.get(f), b.get(f)), f
 
 
+@pytest.mark.parametrize("n, box", [(1, 0.1), (2, 0.05), (40, 0.08), (257, 0.12), (2000, 0.25)])
+def test_springs_carried_over_rebuilds(n, box):
+    """Springs after three rebuilds of the pair lists (none to a few thousand
+    pairs) against the oracle: FP64 forces, 1e-8 as for one evaluation (15
+    steps add rounding of 1e-16 to values that grow by a factor of 15)."""
+    s = random_scene(n=n, seed=n, box=box)
+    o = oracle.OracleDEM(s)
+    g = ts.DEMSceneGPU(s, fp64=True)
+    o.step(15)
+    g.step(15)
+    assert np.array_equal(g.get("objectPointing"), o.get("pointing"))
+    want = np.asarray(o.get("sliding")).reshape(-1)
+    got = np.asarray(g.get("slidingSpring")).reshape(-1)
+    assert got.shape == want.shape
+    if len(want):
+        assert np.abs(got - want).max() <= 1e-8 * max(np.abs(want).max(), 1e-300)
+
+
 def test_clumps_on_plane_match_oracle():
     s = scenes.DEMScene("clumps")
     rng = np.random.default_rng(5)

@@ -286,9 +286,8 @@ struct WritePairsArgs {
     Periodic per;
 };
 
-// writeBallInteractionsKernel (ballNeighborSearchKernel.cu:61-151) with the
-// history carried by insertion indices: a new pair (A,B) takes the springs
-// of the old pair (A,B) if it existed, else zero.
+// writeBallInteractionsKernel (ballNeighborSearchKernel.cu:61-151): the walk
+// writes the partners, k_carry_pairs then the springs.
 template <int L, bool PER>
 __global__ __launch_bounds__(kT) void k_write_pairs(WritePairsArgs a)
 {
@@ -304,13 +303,6 @@ __global__ __launch_bounds__(kT) void k_write_pairs(WritePairsArgs a)
         walk_pair_rows<PER>(a.b, a.g, a.cs, a.ce, i, q0, q1, a.per, [&](int, int) { c++; });
         w += group_exclusive<L>(c, q);
     }
-    const int oa = a.b.orig[i];
-    int os0 = 0, os1 = 0;
-    if (a.has_old) {
-        const int s = a.rank_old[oa];
-        os0 = min(a.old.start[s], a.old.cap);
-        os1 = min(a.old.start[s + 1], a.old.cap);
-    }
     walk_pair_rows<PER>(a.b, a.g, a.cs, a.ce, i, q0, q1, a.per, [&](int j, int code) {
         if (w >= a.cur.cap) {  // over capacity: counted, not stored; the block is replayed
             w++;
@@ -319,9 +311,27 @@ __global__ __launch_bounds__(kT) void k_write_pairs(WritePairsArgs a)
         a.cur.partner[w] = j;
         a.cur.owner[w] = i;
         if (PER) a.cur.shift[w] = (uint8_t)code;
-        double s[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-        const int ob = a.b.orig[j];
-        for (int p = os0; p < os1; p++) {
+        w++;
+    });
+}
+
+// The history of the pairs, carried by insertion indices: a new pair (A,B)
+// takes the springs of the old pair (A,B) if it existed, else zero; and the
+// number of pairs by partner.  One thread a pair: in the walk the search of
+// the old list was a chain of loads behind every pair of a ball, and its 72
+// bytes a pair went out a few lanes at a time (200k balls: 121 us
+// for the walk and 5 for the counts, now 45 and 22; 4k: 33 and 4, now 27 and 5).
+__global__ __launch_bounds__(kT) void k_carry_pairs(WritePairsArgs a, int* rcnt)
+{
+    const int w = xcd_block_spread<8>() * kT + threadIdx.x;
+    if (w >= min(a.cur.start[a.b.n], a.cur.cap)) return;
+    const int j = a.cur.partner[w];
+    atomicAdd(&rcnt[j], 1);
+    double s[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    if (a.has_old) {
+        const int ob = a.b.orig[j], slot = a.rank_old[a.b.orig[a.cur.owner[w]]];
+        const int p1 = min(a.old.start[slot + 1], a.old.cap);
+        for (int p = min(a.old.start[slot], a.old.cap); p < p1; p++) {
             if (a.old_orig[a.old.partner[p]] == ob) {
                 s[0] = a.old.sx[p]; s[1] = a.old.sy[p]; s[2] = a.old.sz[p];
                 s[3] = a.old.rx[p]; s[4] = a.old.ry[p]; s[5] = a.old.rz[p];
@@ -329,22 +339,14 @@ __global__ __launch_bounds__(kT) void k_write_pairs(WritePairsArgs a)
                 break;
             }
         }
-        a.cur.sx[w] = s[0]; a.cur.sy[w] = s[1]; a.cur.sz[w] = s[2];
-        a.cur.rx[w] = s[3]; a.cur.ry[w] = s[4]; a.cur.rz[w] = s[5];
-        a.cur.ox[w] = s[6]; a.cur.oy[w] = s[7]; a.cur.oz[w] = s[8];
-        w++;
-    });
+    }
+    a.cur.sx[w] = s[0]; a.cur.sy[w] = s[1]; a.cur.sz[w] = s[2];
+    a.cur.rx[w] = s[3]; a.cur.ry[w] = s[4]; a.cur.rz[w] = s[5];
+    a.cur.ox[w] = s[6]; a.cur.oy[w] = s[7]; a.cur.oz[w] = s[8];
 }
 
 // Reverse index: pairs grouped by partner, ascending pair id within each
 // partner (the reference sorts pairs by pointing object, DEMSolver.h:59-78).
-__global__ __launch_bounds__(kT) void k_rev_count(int n, const int* start, int cap, const int* partner, int* rcnt)
-{
-    const int i = blockIdx.x * kT + threadIdx.x;
-    if (i >= n) return;
-    const int p1 = min(start[i + 1], cap);
-    for (int p = start[i]; p < p1; p++) atomicAdd(&rcnt[partner[p]], 1);
-}
 __global__ __launch_bounds__(kT) void k_rev_fill(int n, const int* start, int cap, const int* partner,
                                                  const int* rstart, int* rcursor, int* rpair)
 {
@@ -2073,7 +2075,7 @@ struct demsph_dem {
         // reverse index by partner (DEMSolver.h:59-78, reset every build)
         timer.begin("dem_reverse_index", stream);
         // rcnt and rcursor were cleared by k_reorder
-        hipLaunchKernelGGL(k_rev_count, gb, tb, 0, stream, n, pstart[cp].p, pcap[cp], ppartner[cp].p, rcnt.p);
+        hipLaunchKernelGGL(k_carry_pairs, dim3(std::max(1, blocks_for(pcap[cp], kT))), tb, 0, stream, wa, rcnt.p);
         exclusive_scan(rcnt.p, rstart.p, n + 1, scan_temp, nullptr, stream);
         hipLaunchKernelGGL(k_rev_fill, gb, tb, 0, stream, n, pstart[cp].p, pcap[cp], ppartner[cp].p, rstart.p,
                            rcursor.p, rpair.p);
