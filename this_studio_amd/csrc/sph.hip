@@ -2530,8 +2530,8 @@ struct demsph_sph {
     // particles): the fewest of 2, 4, 8 that put 600k threads in flight.
     // More particles a wave share more of its candidate loads, and fewer
     // waves hide less of each other's latencies.  Measured with 8 / 4 / 2
-    // lanes, us: 2k particles 26 / 34 / 54, 18k 29 / 38 / 61, 60k 53 / 54 /
-    // 79, 256k 133 / 117 / 128, 1M 429 / 340 / 314.
+    // lanes, us: 2k particles 26 / 36 / 55, 18k 31 / 39 / 63, 60k 54 / 56 /
+    // 80, 256k 137 / 125 / 134, 1M 443 / 355 / 330.
     int list_lanes() const
     {
         if (list_lanes_set > 0) return list_lanes_set;
