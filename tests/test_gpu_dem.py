@@ -180,6 +180,15 @@ def test_read_back_leaves_the_scene_alone():
         assert np.array_equal(a.get(f), b.get(f)), f
 
 
+def test_fields_read_from_several_threads():
+    """As for the fluid: a read has room of its own, and reads take turns."""
+    from test_gpu_sph import read_from_threads
+
+    g = ts.DEMSceneGPU(random_scene(n=20000, seed=3, box=0.75))
+    g.step(3)
+    assert read_from_threads(g, ["position", "velocity", "force", "radius"], 150) == []
+
+
 @pytest.mark.parametrize("n, box", [(1, 0.1), (2, 0.05), (40, 0.08), (257, 0.12), (2000, 0.25)])
 def test_springs_carried_over_rebuilds(n, box):
     """Springs after three rebuilds of the pair lists (none to a few thousand

@@ -401,6 +401,38 @@ def test_read_back_in_insertion_order(n):
         assert np.array_equal(a.get(f), b.get(f)), f
 
 
+def read_from_threads(scene, fields, rounds):
+    """Fields of one scene read by a thread each, at the same time: the reads
+    that differ from the same fields read in turn."""
+    import threading
+
+    want = {f: scene.get(f) for f in fields}
+    wrong = []
+
+    def reader(f):
+        for k in range(rounds):
+            if not np.array_equal(scene.get(f), want[f]):
+                wrong.append((f, k))
+
+    threads = [threading.Thread(target=reader, args=(f,)) for f in fields]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    return wrong
+
+
+@pytest.mark.parametrize("n", [100, 30000])
+def test_fields_read_from_several_threads(n):
+    rng = np.random.default_rng(n)
+    spec = scenes.SPHSceneSpec(fluid_pos=rng.uniform(0.0, 0.4, (n, 3)), fluid_vel=rng.uniform(-1.0, 1.0, (n, 3)),
+                               dummy_pos=np.zeros((0, 3)), dx=0.01, rho0=1000.0, c0=10.0, nu=1e-6, min_bound=np.zeros(3),
+                               max_bound=np.full(3, 0.4), gravity=np.array([0.0, 0.0, -9.81]), dt=1e-6)
+    s = make_gpu(spec)
+    s.step(spec.dt, 2)
+    assert read_from_threads(s, ["position", "velocity", "density", "densityChange"], 150) == []
+
+
 def test_two_phases_match_oracle():
     """Two fluid phases of different spacing, density and viscosity side by
     side (the kernels' non-uniform paths: per-pair cuts, phase lookups,

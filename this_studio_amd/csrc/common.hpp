@@ -312,44 +312,42 @@ void step_stamp(const StepStamps& st, hipStream_t s);
 
 // -------------------------------------------------------------- read-back
 // Values of sorted particles as doubles in insertion order, COMPS to a
-// particle; the output runs through the parts, n values each.
+// particle.
 template <class T, int COMPS>
 __global__ __launch_bounds__(256) void k_in_order(size_t n, std::array<const T*, 3> src, int stride,
-                                                  const int* __restrict__ orig, double* p0, double* p1, double* p2)
+                                                  const int* __restrict__ orig, double* __restrict__ out)
 {
     const size_t k = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (k >= n) return;
     const size_t o = (size_t)orig[k];
 #pragma unroll
-    for (int c = 0; c < COMPS; c++) {
-        const size_t at = COMPS * o + c;
-        (at < n ? p0[at] : at < 2 * n ? p1[at - n] : p2[at - 2 * n]) = (double)src[c][k * stride];
-    }
+    for (int c = 0; c < COMPS; c++) out[COMPS * o + c] = (double)src[c][k * stride];
 }
-// One kernel puts the values in order in scratch (parts of n doubles,
-// joined if they are one allocation, end to end) and the copies go straight to the caller's memory.  Copying the arrays and their
-// order to the host and scattering them there, on the query for the count as
-// well, was bound by the host.
-// Position and velocity of 2k / 18k / 256k / 1M particles: 0.33 -> 0.10,
-// 0.29 -> 0.10, 3.5 -> 0.74, 18.4 -> 2.7 ms; of 200k balls 2.3 -> 0.59 ms.
+// A scene's room for one field in insertion order, 3 doubles a particle.  A
+// buffer of its own: reading leaves the scene alone, whatever else is queued
+// for it, and reads from several threads take turns on it (the lock is held
+// from the kernel to the end of the copy).
+struct ReadBack {
+    double* buf = nullptr;
+    std::mutex mu;
+};
+// One kernel puts the values in order and one copy takes them to the
+// caller's memory.  Copying the arrays and their order to the host and
+// scattering them there, on the query for the count as well, was bound by
+// the host.  Position and velocity of 2k / 18k / 256k / 1M particles: 0.33 ->
+// 0.09, 0.29 -> 0.10, 3.5 -> 0.72, 18.4 -> 2.75 ms.
 template <class T, int COMPS>
-void read_in_order(size_t n, const std::array<const T*, 3>& src, int stride, const int* orig, double* const (&part)[3],
-                   bool joined, void* out, size_t capacity, size_t* count, hipStream_t st)
+void read_in_order(size_t n, const std::array<const T*, 3>& src, int stride, const int* orig, ReadBack& rb, void* out,
+                   size_t capacity, size_t* count, hipStream_t st)
 {
     if (count) *count = COMPS * n;
     if (!out) return;
     if (capacity < COMPS * n) throw InvalidArg("output capacity too small");
-    if (n) {
-        k_in_order<T, COMPS><<<dim3(blocks_for((long long)n, 256)), dim3(256), 0, st>>>(n, src, stride, orig, part[0],
-                                                                                       part[1], part[2]);
-        DEMSPH_HIP(hipGetLastError());
-        const int parts = joined ? 1 : COMPS;
-        const size_t m = COMPS * n / parts;
-        for (int c = 0; c < parts; c++)
-            DEMSPH_HIP(hipMemcpyAsync(static_cast<double*>(out) + c * m, part[c], m * sizeof(double),
-                                      hipMemcpyDeviceToHost, st));
-    }
-    DEMSPH_HIP(hipStreamSynchronize(st));
+    if (!n) return;
+    std::lock_guard<std::mutex> lk(rb.mu);
+    k_in_order<T, COMPS><<<dim3(blocks_for((long long)n, 256)), dim3(256), 0, st>>>(n, src, stride, orig, rb.buf);
+    DEMSPH_HIP(hipGetLastError());
+    copy_sync(out, rb.buf, COMPS * n * sizeof(double), hipMemcpyDeviceToHost, st);
 }
 
 }  // namespace demsph

@@ -1526,6 +1526,8 @@ struct demsph_dem {
     StepStamps stamps;  // step-end timestamps (batched serving)
 
     // balls: two buffers, cur is the live one
+    DBuf<double> read_room;  // of read_back
+    ReadBack read_back;
     DBuf<double> bpx[2], bpy[2], bpz[2], bvx[2], bvy[2], bvz[2], bwx[2], bwy[2], bwz[2], br[2], bim[2];
     DBuf<int> bmat[2], bclump[2], borig[2];
     int cb = 0;
@@ -1825,6 +1827,7 @@ struct demsph_dem {
         const size_t cells = grid_set(gg, minb, maxb, c) ? (size_t)gg.numGrids() : 0;
         const size_t per_ball = 2 * (11 * 8 + 3 * 4)          // state, two buffers
                                 + 2 * 4 + 12 * 8              // ranks, force and torque accumulators
+                                + 3 * 8                       // read-back
                                 + 5 * 4 + 4 * 4 + 2 * 4       // sort keys, counts and scans, pair starts
                                 + 6 * (2 * (4 + 16 * 8) + 4); // pairs with history (two lists), reverse index
         return nb * per_ball + 2 * cells * sizeof(int) + radix_sort_temp_bytes((int)std::max<size_t>(nb, 1)) +
@@ -1892,6 +1895,8 @@ struct demsph_dem {
         up(bmat[0], hb.mat, n);
         up(bclump[0], hb.clump, n);
         rank.alloc(n); rank_old.alloc(n);
+        read_room.alloc(3 * (size_t)n);
+        read_back.buf = read_room.p;
         iota_i32(borig[0].p, n, stream);
         iota_i32(rank.p, n, stream);
         for (auto* d : {&fx, &fy, &fz, &tx, &ty, &tz}) d->alloc(n);
@@ -3128,13 +3133,11 @@ extern "C" int demsph_dem_get(demsph_dem* d, const char* field, void* out, size_
         hipStream_t st = d->stream;
         const int cb = d->cb;
         const size_t n = d->n;
-        // the copies that the next sort fills are free between calls
-        double* const part[3] = {d->bpx[1 - cb].p, d->bpy[1 - cb].p, d->bpz[1 - cb].p};
         auto vec = [&](const DBuf<double>& x, const DBuf<double>& y, const DBuf<double>& z) {
-            read_in_order<double, 3>(n, {x.p, y.p, z.p}, 1, d->borig[cb].p, part, false, out, capacity, count, st);
+            read_in_order<double, 3>(n, {x.p, y.p, z.p}, 1, d->borig[cb].p, d->read_back, out, capacity, count, st);
         };
         auto scal = [&](const DBuf<double>& x) {
-            read_in_order<double, 1>(n, {x.p}, 1, d->borig[cb].p, part, false, out, capacity, count, st);
+            read_in_order<double, 1>(n, {x.p}, 1, d->borig[cb].p, d->read_back, out, capacity, count, st);
         };
         auto plain3 = [&](const DBuf<double>& x, const DBuf<double>& y, const DBuf<double>& z, size_t m) {
             auto hx = fetch(x.p, m, st), hy = fetch(y.p, m, st), hz = fetch(z.p, m, st);

@@ -2128,6 +2128,7 @@ struct demsph_sph {
     int* maxcount = nullptr;      // device [2]
     int* maxcount_h = nullptr;    // pinned [2]
     bool lists_valid = false;
+    ReadBack read_back;
     // 32-byte gather records (uniform scenes): knob, state, the two buffers
     // the passes of a step alternate between
     bool pair_records = true;
@@ -2203,7 +2204,7 @@ struct demsph_sph {
         sort_temp = nullptr;
         dfree(cells); dfree(nbr_ff); dfree(cnt_ff); dfree(nbr_fd); dfree(cnt_fd); dfree(DA); dfree(DB); dfree(DC);
         dfree(GR[0]); dfree(GR[1]);
-        dfree(maxcount);
+        dfree(maxcount); dfree(read_back.buf);
         host_free(maxcount_h);
         maxcount_h = nullptr;
         dfree(DP); dfree(DV); dfree(dphase); dfree(dorig); dfree(dcells); dfree(dummy_near); dfree(d_phases);
@@ -2304,6 +2305,7 @@ struct demsph_sph {
         const size_t per_fluid = 2 * rec + rec + sizeof(int)             // two buffers, checkpoint, rank
                                  + 2 * sizeof(GRec)                       // gather records
                                  + 2 * sizeof(int)                        // list counts
+                                 + 3 * sizeof(double)                     // read-back
                                  + sizeof(int) * (size_t)(round_chunk(K_ff) + round_chunk(K_fd));
         const size_t per_sort = 3 * sizeof(uint32_t) + 2 * sizeof(int);
         const size_t per_dummy = sizeof(DummyPos) + 3 * sizeof(float4) + sizeof(float2) + 1 + sizeof(int);
@@ -2378,6 +2380,7 @@ struct demsph_sph {
         }
         cnt_ff = dmalloc<int>(n); cnt_fd = dmalloc<int>(n);
         GR[0] = dmalloc<GRec>(n); GR[1] = dmalloc<GRec>(n);
+        read_back.buf = dmalloc<double>(3 * n);
         maxcount = dmalloc<int>(3);
         DEMSPH_HIP(host_malloc((void**)&maxcount_h, 3 * sizeof(int)));
         alloc_lists();
@@ -3206,21 +3209,18 @@ extern "C" int demsph_sph_get(demsph_sph* s, const char* field, void* out, size_
         const std::string f = field;
         hipStream_t st = s->stream;
         const size_t n = s->nf;
-        // the buffer that the next pass overwrites is free between calls
         const int* const to = s->orig[s->cO];
         const FluidPos* const P = s->P[s->cP];
-        double* const w = reinterpret_cast<double*>(s->P[1 - s->cP]);
-        static_assert(sizeof(FluidPos) == 4 * sizeof(double), "a record holds the three components");
-        double* const part[3] = {w, w + n, w + 2 * n};
+        ReadBack& rb = s->read_back;
         if (f == "position")
-            return read_in_order<double, 3>(n, {&P->x, &P->y, &P->z}, 4, to, part, true, out, capacity, count, st);
-        if (f == "density") return read_in_order<float, 1>(n, {&P->rho}, 8, to, part, true, out, capacity, count, st);
-        if (f == "pressure") return read_in_order<float, 1>(n, {&P->p}, 8, to, part, true, out, capacity, count, st);
+            return read_in_order<double, 3>(n, {&P->x, &P->y, &P->z}, 4, to, rb, out, capacity, count, st);
+        if (f == "density") return read_in_order<float, 1>(n, {&P->rho}, 8, to, rb, out, capacity, count, st);
+        if (f == "pressure") return read_in_order<float, 1>(n, {&P->p}, 8, to, rb, out, capacity, count, st);
         if (f == "velocity")
-            return read_in_order<double, 3>(n, {s->vx[s->cV], s->vy[s->cV], s->vz[s->cV]}, 1, to, part, true, out, capacity,
+            return read_in_order<double, 3>(n, {s->vx[s->cV], s->vy[s->cV], s->vz[s->cV]}, 1, to, rb, out, capacity,
                                             count, st);
         if (f == "densityChange")
-            return read_in_order<float, 1>(n, {s->drho[s->cD]}, 1, to, part, true, out, capacity, count, st);
+            return read_in_order<float, 1>(n, {s->drho[s->cD]}, 1, to, rb, out, capacity, count, st);
         auto orig = fetch(to, n, st);
         if (f == "dummyNormal") {
             const size_t m = s->nd;
