@@ -106,7 +106,10 @@ void o_cell_ranges(const int* sh, int n, int numGrids, int* start, int* end)
     }
 }
 
-/* ballNeighborSearchKernel.cu:23-33 / SPHNeighborSearchKernel.cu:21-31 */
+/* ballNeighborSearchKernel.cu:23-33 / SPHNeighborSearchKernel.cu:21-31.  On an
+ * axis of one cell a point at or past the maximum face shrinks on both sides:
+ * the reference leaves it the cell before the only one, which is another
+ * row's cell or none of the array. */
 void o_stencil(const o_grid* g, const double* p, int* cell, int* lo, int* hi)
 {
     int gx = (int)((p[0] - g->minx) / g->cx);
@@ -115,11 +118,11 @@ void o_stencil(const o_grid* g, const double* p, int* cell, int* lo, int* hi)
     lo[0] = lo[1] = lo[2] = -1;
     hi[0] = hi[1] = hi[2] = 1;
     if (gx <= 0) { gx = 0; lo[0] = 0; }
-    if (gx >= g->nx - 1) { gx = g->nx - 1; hi[0] = 0; }
+    if (gx >= g->nx - 1) { gx = g->nx - 1; hi[0] = 0; if (gx == 0) lo[0] = 0; }
     if (gy <= 0) { gy = 0; lo[1] = 0; }
-    if (gy >= g->ny - 1) { gy = g->ny - 1; hi[1] = 0; }
+    if (gy >= g->ny - 1) { gy = g->ny - 1; hi[1] = 0; if (gy == 0) lo[1] = 0; }
     if (gz <= 0) { gz = 0; lo[2] = 0; }
-    if (gz >= g->nz - 1) { gz = g->nz - 1; hi[2] = 0; }
+    if (gz >= g->nz - 1) { gz = g->nz - 1; hi[2] = 0; if (gz == 0) lo[2] = 0; }
     cell[0] = gx; cell[1] = gy; cell[2] = gz;
 }
 

@@ -189,6 +189,23 @@ def test_fields_read_from_several_threads():
     assert read_from_threads(g, ["position", "velocity", "force", "radius"], 150) == []
 
 
+@pytest.mark.parametrize("thin", [(0,), (1,), (2,), (0, 1, 2)])
+def test_pairs_on_axes_of_one_cell(thin):
+    """Pair lists in domains of one cell on some axes, balls past the faces and
+    on them, at every lane count."""
+    s = random_scene(n=400, seed=thin[0] + len(thin), box=0.12)
+    s.max_bound[list(thin)] = 0.03
+    o = oracle.OracleDEM(s)
+    for lanes in (1, 2, 4, 8):
+        g = ts.DEMSceneGPU(s)
+        g.tune("pairLanes", lanes)
+        g.neighbor_search()
+        if lanes == 1:
+            o.neighbor_search()
+        assert np.array_equal(g.get("objectPointed"), o.get("pointed")), lanes
+        assert np.array_equal(g.get("objectPointing"), o.get("pointing")), lanes
+
+
 @pytest.mark.parametrize("n, box", [(1, 0.1), (2, 0.05), (40, 0.08), (257, 0.12), (2000, 0.25)])
 def test_springs_carried_over_rebuilds(n, box):
     """Springs after three rebuilds of the pair lists (none to a few thousand

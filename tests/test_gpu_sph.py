@@ -348,6 +348,39 @@ def test_lists_at_slot_edges_and_outside_the_grid(n, two_h):
         assert np.array_equal(s.get("dummyObjectPointing"), o.get("pointing_fd")), L
 
 
+@pytest.mark.parametrize("thin", [(0,), (1,), (2,), (0, 1), (0, 2), (1, 2), (0, 1, 2)])
+def test_lists_on_axes_of_one_cell(thin):
+    """Domains of one cell on some axes, of 1.4 supports, with particles and
+    dummies past the faces and on them: fluid and dummy lists and the dummy
+    normals (1e-6 on unit vectors in FP32) against the oracle."""
+    rng = np.random.default_rng(10 * len(thin) + thin[0])
+    dx = 0.01
+    cut = 2.0 * 1.3 * dx
+    side = np.full(3, 3.3 * cut)
+    side[list(thin)] = 1.4 * cut
+
+    def points(n):
+        p = rng.uniform(0.0, 1.0, (n, 3)) * side
+        off = rng.random((n, 3))
+        p += np.where(off < 0.1, -1.0, np.where(off > 0.85, 1.0, 0.0)) * rng.uniform(0.0, 1.5, (n, 3)) * cut
+        for k in range(3):
+            p[10 * k:10 * k + 10, k] = side[k]
+        return p
+
+    spec = scenes.SPHSceneSpec(fluid_pos=points(400), dummy_pos=points(200), dx=dx, rho0=1000.0, c0=10.0, nu=1e-6,
+                               min_bound=np.zeros(3), max_bound=side, gravity=np.array([0.0, 0.0, -9.81]), dt=1e-5)
+    o = oracle.OracleSPH(spec)
+    o.neighbor_search()
+    s = make_gpu(spec)
+    s.neighbor_search()
+    assert np.array_equal(s.get("hashIndex"), o.get("index"))
+    assert np.array_equal(s.get("neighborCount"), o.get("count_ff"))
+    assert np.array_equal(s.get("objectPointing"), o.get("pointing_ff"))
+    assert np.array_equal(s.get("dummyNeighborCount"), o.get("count_fd"))
+    assert np.array_equal(s.get("dummyObjectPointing"), o.get("pointing_fd"))
+    np.testing.assert_allclose(s.get("dummyNormal"), o.get("dnormal"), atol=1e-6)
+
+
 @pytest.mark.parametrize("field", ["velocity", "densityChange"])
 def test_records_follow_a_field_set_between_search_and_halves(field, small):
     """A field set after the search reaches the records that the passes

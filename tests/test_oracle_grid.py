@@ -108,3 +108,37 @@ def test_sph_pair_set_independent_of_cell_size():
         cnt, pa, pb = _pairs_oracle(g, pos, h)
         sets.append(set(zip(pa.tolist(), pb.tolist())))
     assert sets[0] == sets[1] == sets[2]
+
+
+@pytest.mark.parametrize("counts", [(1, 1, 1), (1, 3, 2), (4, 1, 3), (2, 3, 1), (5, 1, 1)])
+def test_stencil_stays_in_the_grid(counts):
+    """Stencils of points in, on and far past every face hold cells of the grid
+    only, on axes of one cell too, and the lists of such points are those of
+    brute force over particles whose cells the stencils meet."""
+    side = np.array(counts, dtype=float)
+    g = oracle.grid_set([0, 0, 0], side, 1.0)
+    assert (g.nx, g.ny, g.nz) == counts
+    rng = np.random.default_rng(sum(counts))
+    n = 400
+    pos = rng.uniform(0.0, side, (n, 3))
+    out = rng.random((n, 3))
+    pos += np.where(out < 0.15, -rng.uniform(0, 3, (n, 3)), np.where(out > 0.85, rng.uniform(0, 3, (n, 3)), 0.0))
+    pos[:20, 0] = side[0]  # on the maximum faces
+    pos[10:30, 1] = side[1]
+    dims = np.array(counts)
+    cells, lo, hi = (np.zeros((n, 3), dtype=np.int32) for _ in range(3))
+    for k in range(n):
+        oracle.lib().o_stencil(oracle.Grid.from_buffer_copy(g), oracle.d(pos[k].copy()), oracle.i(cells[k]), oracle.i(lo[k]),
+                               oracle.i(hi[k]))
+    assert (cells + lo >= 0).all() and (cells + hi < dims).all() and (lo <= hi).all()
+    hv = oracle.hash_points(g, pos)
+    home = np.stack([hv % dims[0], hv // dims[0] % dims[1], hv // (dims[0] * dims[1])], -1)
+    h = np.full(n, 0.4)
+    cnt, pa, pb = _pairs_oracle(g, pos, h)
+    d2 = ((pos[:, None] - pos[None]) ** 2).sum(-1)
+    step = home[None] - cells[:, None]
+    met = ((step >= lo[:, None]) & (step <= hi[:, None])).all(-1)
+    mask = met & (0.8 * 0.8 - d2 >= 0)
+    np.fill_diagonal(mask, False)
+    assert np.array_equal(cnt, mask.sum(1))
+    assert set(zip(pa.tolist(), pb.tolist())) == {(int(a), int(b)) for a, b in zip(*np.nonzero(mask))}

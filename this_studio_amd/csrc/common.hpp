@@ -211,7 +211,9 @@ __device__ __forceinline__ int cell_hash(const GridGeom& g, double px, double py
 
 // 27-cell stencil of a query point (ballNeighborSearchKernel.cu:23-33,
 // SPHNeighborSearchKernel.cu:21-31): unclamped truncation, grid clamp and
-// face shrink.
+// face shrink.  On an axis of one cell a point at or past the maximum face
+// shrinks on both sides: the reference leaves it the cell before the only
+// one, which is another row's cell or none of the array.
 struct Stencil {
     int cx, cy, cz;
     int lox, loy, loz, hix, hiy, hiz;
@@ -226,11 +228,11 @@ __device__ __forceinline__ Stencil make_stencil(const GridGeom& g, double px, do
     s.lox = s.loy = s.loz = -1;
     s.hix = s.hiy = s.hiz = 1;
     if (gx <= 0) { gx = 0; s.lox = 0; }
-    if (gx >= g.nx - 1) { gx = g.nx - 1; s.hix = 0; }
+    if (gx >= g.nx - 1) { gx = g.nx - 1; s.hix = 0; if (gx == 0) s.lox = 0; }
     if (gy <= 0) { gy = 0; s.loy = 0; }
-    if (gy >= g.ny - 1) { gy = g.ny - 1; s.hiy = 0; }
+    if (gy >= g.ny - 1) { gy = g.ny - 1; s.hiy = 0; if (gy == 0) s.loy = 0; }
     if (gz <= 0) { gz = 0; s.loz = 0; }
-    if (gz >= g.nz - 1) { gz = g.nz - 1; s.hiz = 0; }
+    if (gz >= g.nz - 1) { gz = g.nz - 1; s.hiz = 0; if (gz == 0) s.loz = 0; }
     s.cx = gx; s.cy = gy; s.cz = gz;
     return s;
 }
