@@ -381,6 +381,44 @@ def test_lists_on_axes_of_one_cell(thin):
     np.testing.assert_allclose(s.get("dummyNormal"), o.get("dnormal"), atol=1e-6)
 
 
+@pytest.mark.parametrize("two_h", [False, True])
+@pytest.mark.parametrize("side", [0.3, 0.5, 0.7, 0.95])
+def test_lists_in_a_domain_smaller_than_a_support(side, two_h):
+    """A domain of `side` supports on every axis is one cell whose edges are
+    shorter than the cut.  Particles up to 30 of these edges outside it,
+    thickest at 8 to 14 of them: lists equal the oracle's at every lane
+    count."""
+    rng = np.random.default_rng(int(100 * side))
+    dx = 0.01
+    cut = 2.0 * 1.3 * dx
+    edge = side * cut
+    pos = [rng.uniform(0.0, edge, (20, 3))]
+    for d in np.concatenate([np.arange(8.0, 14.0, 0.25), rng.uniform(0.0, 30.0, 20)]):
+        c = rng.uniform(0.0, edge, 3)
+        c[rng.integers(3)] += edge * d * rng.choice([-1.0, 1.0])
+        pos.append(c + rng.uniform(-0.4, 0.4, (6, 3)) * cut)
+    # a line of close neighbours through all of the limits
+    t = np.arange(-16.0 * edge, 17.0 * edge, 0.3 * cut)
+    pos.append(np.stack([t, np.full(len(t), 0.5 * edge), np.full(len(t), 0.4 * edge)], -1))
+    pos = np.concatenate(pos)
+    g = np.arange(-15.0 * edge, 16.0 * edge, 0.5 * cut)
+    dummy = np.stack([g, np.full(len(g), 0.6 * edge), np.full(len(g), 0.3 * edge)], -1)
+    spec = scenes.SPHSceneSpec(fluid_pos=pos, dummy_pos=dummy, dx=dx, rho0=1000.0, c0=10.0, nu=1e-6, min_bound=np.zeros(3),
+                               max_bound=np.full(3, edge), gravity=np.array([0.0, 0.0, -9.81]), dt=1e-5)
+    if two_h:
+        spec.fluid_dx = np.where(rng.random(len(pos)) < 0.5, dx, 0.8 * dx)
+    o = oracle.OracleSPH(spec)
+    o.neighbor_search()
+    for L in (0, 1, 2, 4, 8):
+        s = make_gpu(spec)
+        s.tune("listLanes", L)
+        s.neighbor_search()
+        assert np.array_equal(s.get("neighborCount"), o.get("count_ff")), L
+        assert np.array_equal(s.get("objectPointing"), o.get("pointing_ff")), L
+        assert np.array_equal(s.get("dummyNeighborCount"), o.get("count_fd")), L
+        assert np.array_equal(s.get("dummyObjectPointing"), o.get("pointing_fd")), L
+
+
 @pytest.mark.parametrize("field", ["velocity", "densityChange"])
 def test_records_follow_a_field_set_between_search_and_halves(field, small):
     """A field set after the search reaches the records that the passes

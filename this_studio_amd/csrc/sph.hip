@@ -84,28 +84,31 @@ struct alignas(32) SolidPos {
 static_assert(sizeof(SolidPos) == 32, "SolidPos is one 32-byte record");
 
 // Fixed-point positions.  A coordinate is stored as the low 32 bits of
-// round((x - min) / u), with 2^25 to 2^26 units u to the largest cell edge:
-// positions modulo 64 cells or more, at most 3e-8 cells (8e-8 spacings) apart.  Everything that compares two
+// round((x - min) / u), with 2^25 to 2^26 units u to an edge: the largest
+// cell edge, or the largest cut where a domain smaller than that on every
+// axis has shorter cells.  That is positions modulo 64 edges or more, at most
+// 3e-8 edges (8e-8 spacings) apart.  Everything that compares two
 // positions meets them within one 27-cell stencil, where the wrapped 32-bit
 // difference is the true one, exact to one unit however large the grid: an
 // integer subtraction and a conversion where offsets from cell origins took
 // the neighbour's cell out of the list entry and nine FP32 operations.
 //
-// A point is "far" when that argument does not cover it: more than 10.5 cells
+// A point is "far" when that argument does not cover it: more than 10.5 edges
 // outside the grid on some axis (its hash is clamped into the face cells; 12
-// cells on both sides plus a stencil stay far below the 64-cell period), on
+// edges on both sides plus a stencil stay far below the 64-edge period), on
 // the rounding edge of the maximum face (where the hash can land in another
 // row of cells), or not a number.  Far points take the FP64 test in the list
 // build, and a particle that is far or lists a far neighbour takes the FP64
-// records in the pair passes (kFarBit of its count).  Beyond 12 cells, or not
+// records in the pair passes (kFarBit of its count).  Beyond 12 edges, or not
 // a number, it is "out": farther than any cut from every point that is not far.
-constexpr double kFixPerCell = 67108864.0;  // 2^26: units to a cell edge, at most
-constexpr double kFixPad = 12.0 * kFixPerCell, kFixNear = 10.5 * kFixPerCell;
+constexpr double kFixPerEdge = 67108864.0;  // 2^26: units to an edge, at most
+constexpr double kFixPad = 12.0 * kFixPerEdge, kFixNear = 10.5 * kFixPerEdge;
 struct FixGeom {
     double minx, miny, minz;
     double ex, ey, ez;  // extent of the grid in units
     double inv;         // units per metre
     float u;            // metres per unit
+    double edge;        // the edge, in units
 };
 struct Fix3 {
     int x, y, z;
@@ -596,7 +599,7 @@ __device__ __forceinline__ int nth_bit(unsigned m, int n)
 // pair near the cut has |b| <= B = A + c, and its test at most three roundings
 // of 2^-24 B^2, three of B^2 + 2 A B, three of A^2 and one of A^2 + c^2: half
 // the bound that list_error takes.  Candidates farther off (outside the
-// grid, 15 cells at most, or out as FixGeom has it) are off by less than
+// grid, 15 edges at most, or out as FixGeom has it) are off by less than
 // 1e-6 of |b|^2 and clear of the cut by more.
 // Any other particle is a set by itself about its own position, and also
 // takes the exact test against far candidates; one that is out takes no
@@ -1735,7 +1738,7 @@ __global__ __launch_bounds__(256) void k_fs_rev_walk(RevArgs a)
     int off = COUNT ? 0 : a.rstart[j];
     const Fix3 bq = fix_pos(a.fix, bx, by, bz);
     float lo, hi;
-    // differences of up to 27 cells in FP32: 64 units a coordinate
+    // differences of up to 27 edges in FP32: 64 units a coordinate
     cut_band(2.0 * a.hf * a.fix.inv, a.prefilter && !bq.far, 256.0f, 0.0f, lo, hi);
     for (int k = 0; k < 9; k++) {
         const int dz = k / 3 - 1, dy = k % 3 - 1;
@@ -2328,7 +2331,8 @@ struct demsph_sph {
         nf = (int)hf.size();
         nd = (int)hd.size();
         if (nf == 0) throw InvalidArg("no fluid particles");
-        if (!grid_set(grid, minb, maxb, staged_cell_size())) throw InvalidArg("degenerate domain or smoothing length");
+        const double cell = staged_cell_size();
+        if (!grid_set(grid, minb, maxb, cell)) throw InvalidArg("degenerate domain or smoothing length");
         numGrids = grid.numGrids();
         if (numGrids > INT32_MAX / 2) throw InvalidArg("grid too large");
 
@@ -2371,8 +2375,10 @@ struct demsph_sph {
             fix.minx = grid.minx; fix.miny = grid.miny; fix.minz = grid.minz;
             // a power of two of units to the fluid's 2 h makes the kernel
             // argument r / 2h exact in the pair passes
-            const double cmax = std::max(grid.cx, std::max(grid.cy, grid.cz)), two_h = 1.0 / grad_k(phf.hf).half_invh;
-            fix.inv = two_h <= cmax && cmax <= 2.0 * two_h ? 0.5 * kFixPerCell / two_h : kFixPerCell / cmax;
+            const double emax = std::max(std::max(grid.cx, cell), std::max(grid.cy, grid.cz)),
+                         two_h = 1.0 / grad_k(phf.hf).half_invh;
+            fix.inv = two_h <= emax && emax <= 2.0 * two_h ? 0.5 * kFixPerEdge / two_h : kFixPerEdge / emax;
+            fix.edge = emax * fix.inv;
             fix.u = (float)(1.0 / fix.inv);
             fix.ex = (grid.maxx - grid.minx) * fix.inv;
             fix.ey = (grid.maxy - grid.miny) * fix.inv;
@@ -2513,9 +2519,8 @@ struct demsph_sph {
         la.nbr_ff = nbr_ff; la.cnt_ff = cnt_ff; la.nbr_fd = nbr_fd; la.cnt_fd = cnt_fd;
         la.K_ff = K_ff; la.K_fd = K_fd; la.maxcount = maxcount;
         la.A = gr(0); la.DA = DA; la.skey = skey; la.numGrids = numGrids;
-        const double edge = std::max(grid.cx, std::max(grid.cy, grid.cz)) * fix.inv;
-        la.reach = (float)(0.75 * edge);
-        la.err = list_error(la.reach, edge);
+        la.reach = (float)(0.75 * fix.edge);
+        la.err = list_error(la.reach, fix.edge);
         cut_band(2.0 * phf.h * fix.inv, prefilter, kListSlack, la.err, la.lo_f, la.hi_f);
         cut_band(2.0 * std::max(phf.h, phd.h) * fix.inv, prefilter, kListSlack, la.err, la.lo_d, la.hi_d);
         la.stepx = (unsigned long long)(grid.cx * fix.inv * 1048576.0 + 0.5);
