@@ -419,6 +419,47 @@ def test_lists_in_a_domain_smaller_than_a_support(side, two_h):
         assert np.array_equal(s.get("dummyObjectPointing"), o.get("pointing_fd")), L
 
 
+@pytest.mark.parametrize("ops", [
+    ["search", "search", "step", "first", "second", "step"],
+    ["search", "first", "step", "second"],
+    ["search", "first", "second", "step", "first", "second"],
+    ["step", "first", "step", "velocity", "first", "second"],
+])
+def test_halves_after_replayed_blocks(ops, small):
+    """Searches and halves between replays of captured step graphs, at every
+    parity of the buffers that the sequence passes through (its fourth round
+    replays graphs captured in the earlier ones): bit for bit what eager steps
+    give, and within the rounding of the two forms of the pair passes (1e-5 of
+    the largest value, as above) of the FP64 records."""
+    rng = np.random.default_rng(5)
+    kick = 0.05 * rng.uniform(-1.0, 1.0, (small.nf, 3))
+    runs = []
+    for graphs, rec in ((True, 1), (False, 1), (True, 0)):
+        s = make_gpu(small)
+        s.set_graphs(graphs)
+        s.tune("pairRecords", rec)
+        s.step(small.dt, 2)
+        for _ in range(4):
+            for op in ops:
+                if op == "search":
+                    s.neighbor_search()
+                elif op == "first":
+                    s.first_half(small.dt)
+                elif op == "second":
+                    s.second_half(small.dt)
+                elif op == "velocity":
+                    s.set("velocity", s.get("velocity") + kick)
+                else:
+                    s.step(small.dt, 2)
+        s.first_half(small.dt)
+        s.second_half(small.dt)
+        assert (s.graph_captures() > 0) == graphs
+        runs.append([s.get(f) for f in ("position", "velocity", "densityChange")])
+    for a, b, c in zip(*runs):
+        assert np.array_equal(a, b)
+        assert np.abs(a - c).max() < 1e-5 * np.abs(c).max()
+
+
 @pytest.mark.parametrize("field", ["velocity", "densityChange"])
 def test_records_follow_a_field_set_between_search_and_halves(field, small):
     """A field set after the search reaches the records that the passes

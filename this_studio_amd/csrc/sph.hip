@@ -2659,6 +2659,12 @@ struct demsph_sph {
             cG ^= 1;
         }
     }
+    // The records hold no pass's state: none until the next search.
+    void drop_records()
+    {
+        rec_ready = false;
+        cG = 0;
+    }
     // After a host write to the state the records follow it.
     void refresh_records()
     {
@@ -2695,7 +2701,7 @@ struct demsph_sph {
         use_records(a, false);
         // the velocities change and the records do not: a further half
         // before the next search takes the FP64 records
-        rec_ready = false;
+        drop_records();
         if (uniform) momentum_lanes<false, true>("sph_momentum_second", a);
         else momentum_lanes<false, false>("sph_momentum_second", a);
         cV ^= 1;
@@ -2798,6 +2804,7 @@ struct demsph_sph {
         for (auto& e : graphs)
             if (e.key == key) return e.exec;
         const int sP = cP, sV = cV, sD = cD, sO = cO;
+        const bool slists = lists_valid;
         hipGraph_t g = nullptr;
         // No other thread may allocate, free or synchronise the device
         // until the graph is instantiated (see capture_lock).
@@ -2810,6 +2817,8 @@ struct demsph_sph {
             (void)hipStreamEndCapture(stream, &g);
             if (g) (void)hipGraphDestroy(g);
             cP = sP; cV = sV; cD = sD; cO = sO;
+            lists_valid = slists;
+            drop_records();
             throw;
         }
         DEMSPH_HIP(hipStreamEndCapture(stream, &g));
@@ -2839,7 +2848,10 @@ struct demsph_sph {
         int k = 0;
         if (use_graphs && !timer.enabled) {
             if (!cells_track_skey && k < nsteps) { one_step(dt); k++; }
-            for (; k + 2 <= nsteps; k += 2) DEMSPH_HIP(hipGraphLaunch(pair_graph(dt), stream));
+            for (; k + 2 <= nsteps; k += 2) {
+                DEMSPH_HIP(hipGraphLaunch(pair_graph(dt), stream));
+                drop_records();  // a replay runs none of the host's side of its steps
+            }
         }
         for (; k < nsteps; k++) one_step(dt);
     }
