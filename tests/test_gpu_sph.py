@@ -460,6 +460,35 @@ def test_halves_after_replayed_blocks(ops, small):
         assert np.abs(a - c).max() < 1e-5 * np.abs(c).max()
 
 
+@pytest.mark.parametrize("cells", [0.5, 20.0, 64.0, 128.0, 1e6])
+@pytest.mark.parametrize("n", [2, 300])
+def test_a_particle_that_flies_off_in_one_step(n, cells):
+    """One particle drifts `cells` supports in the first half (64 and 128 are
+    multiples of the period of the records' positions), after which the second
+    half must not see it beside its former neighbours.  Records against the
+    FP64 records over the other particles: rounding of FP32 sums, 1e-5 of the
+    largest value."""
+    rng = np.random.default_rng(n)
+    dx, dt = 0.01, 1e-4
+    side = max(0.1, 0.8 * dx * n ** (1.0 / 3.0))
+    pos = 0.5 * side + rng.uniform(-0.5, 0.5, (n, 3)) * (0.4 * dx if n == 2 else side)
+    vel = rng.uniform(-0.1, 0.1, (n, 3))
+    vel[0, 0] = cells * 2.0 * 1.3 * dx / dt
+    spec = scenes.SPHSceneSpec(fluid_pos=pos, fluid_vel=vel, dummy_pos=np.zeros((0, 3)), dx=dx, rho0=1000.0, c0=10.0,
+                               nu=0.0, min_bound=np.zeros(3), max_bound=np.full(3, side),
+                               gravity=np.array([0.0, 0.0, -9.81]), dt=dt)
+    got = []
+    for rec in (1, 0):
+        s = make_gpu(spec)
+        s.tune("pairRecords", rec)
+        s.neighbor_search()
+        s.first_half(dt)
+        s.second_half(dt)
+        got.append([s.get(f)[1:] for f in ("position", "velocity", "densityChange")])
+    for a, b in zip(*got):
+        assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max()
+
+
 @pytest.mark.parametrize("field", ["velocity", "densityChange"])
 def test_records_follow_a_field_set_between_search_and_halves(field, small):
     """A field set after the search reaches the records that the passes

@@ -101,7 +101,14 @@ static_assert(sizeof(SolidPos) == 32, "SolidPos is one 32-byte record");
 // build, and a particle that is far or lists a far neighbour takes the FP64
 // records in the pair passes (kFarBit of its count).  Beyond 12 edges, or not
 // a number, it is "out": farther than any cut from every point that is not far.
+//
+// The drift of the first half moves the points between the search and the
+// passes after it.  Two neighbours' difference stays below 32 edges as long as
+// neither moves more than kFixDrift (15 edges); if any point does, or turns
+// into no number, a flag sends all particles to the FP64 records until the next
+// search (SphArgs::strayed).
 constexpr double kFixPerEdge = 67108864.0;  // 2^26: units to an edge, at most
+constexpr double kFixDrift = 15.0 * kFixPerEdge;
 constexpr double kFixPad = 12.0 * kFixPerEdge, kFixNear = 10.5 * kFixPerEdge;
 struct FixGeom {
     double minx, miny, minz;
@@ -209,6 +216,8 @@ struct SphArgs {
     const float4* GRin;  // split halves, nf float4 apart
     float4* GRout;
     FixGeom fix;
+    int* strayed;    // set by the first half's pass when a point moves farther than records allow
+    float stray_vel;  // velocity above which it does (sum over the axes)
     // fluid and dummy pairs on records: u / 2h, u m_j times the kernel constant (GradK)
     float ff_half_invh, ff_coef, fd_half_invh, fd_coef;
     // dummies (sorted once)
@@ -412,6 +421,7 @@ struct ReorderArgs {
     int2* cells;  // (start, end) per cell
     FixGeom fix;
     float4* oGR;   // records (split halves, n apart)
+    int* strayed;  // cleared
     int rec_full;  // the pair passes gather records: write the second half too
 };
 
@@ -422,6 +432,7 @@ __global__ __launch_bounds__(kThreads) void k_reorder(ReorderArgs a)
     const int o = a.perm[k];
     const int s = a.rank[o];
     a.rank[o] = k;
+    if (k == 0) *a.strayed = 0;
     a.orig_out[k] = o;
     const FluidPos p = a.P[s];
     a.oP[k] = p;
@@ -1298,7 +1309,10 @@ __device__ __forceinline__ void momentum_finish(const SphArgs& a, int i, int q, 
         o.rho = s.rho;
         o.p = s.p;
         a.oP[i] = o;
-        if (a.GRout) st_grec(a.GRout, a.nf, i, a.fix, o, nV);
+        if (a.GRout) {
+            st_grec(a.GRout, a.nf, i, a.fix, o, nV);
+            if (!(fabsf(nV.x) + fabsf(nV.y) + fabsf(nV.z) < a.stray_vel)) *a.strayed = 1;
+        }
     }
 }
 
@@ -1456,9 +1470,9 @@ __global__ __launch_bounds__(kThreads) void k_momentum(SphArgs a)
         static_assert(UNIF && LANES >= 2, "gather records: uniform scenes, entry-split lanes");
         const int cf = a.cnt_ff[i], cd = a.nd > 0 ? a.cnt_fd[i] : 0;
         const int nf = min(list_count(cf), a.K_ff), nd = min(list_count(cd), a.K_fd);
-        if ((cf | cd) & kFarBit) {
-            momentum_far<LANES>(a, i, q, nf, nd, ax, ay, az);
-        } else {
+        const int strayed = FIRST ? 0 : *a.strayed;  // used after the records: its load hides behind them
+        const bool far = (cf | cd) & kFarBit;
+        if (!far) {
             int pre[kPreEntries];
             preload_entries<LANES>(a.nbr_ff, a.K_ff, i, q, pre);
             const PairSelf s = pair_self_rec(a, i);
@@ -1480,6 +1494,10 @@ __global__ __launch_bounds__(kThreads) void k_momentum(SphArgs a)
                 ay += kvd * w.vy - kd * w.py;
                 az += kvd * w.vz - kd * w.pz;
             }
+        }
+        if (__builtin_expect(far || strayed, 0)) {
+            ax = ay = az = 0.f;
+            momentum_far<LANES>(a, i, q, nf, nd, ax, ay, az);
         }
     } else {
         const PairSelf s = pair_self<UNIF>(a, i);
@@ -1605,9 +1623,9 @@ __global__ __launch_bounds__(kThreads) void k_continuity(SphArgs a)
         static_assert(UNIF && LANES >= 2, "gather records: uniform scenes, entry-split lanes");
         const int cf = a.cnt_ff[i], cd = a.nd > 0 ? a.cnt_fd[i] : 0;
         const int nf = min(list_count(cf), a.K_ff), nd = min(list_count(cd), a.K_fd);
-        if ((cf | cd) & kFarBit) {
-            d = continuity_far<LANES>(a, i, q, nf, nd);
-        } else {
+        const int strayed = *a.strayed;
+        const bool far = (cf | cd) & kFarBit;
+        if (!far) {
             int pre[kPreEntries];
             preload_entries<LANES>(a.nbr_ff, a.K_ff, i, q, pre);
             const PairSelf s = pair_self_rec(a, i);
@@ -1623,6 +1641,7 @@ __global__ __launch_bounds__(kThreads) void k_continuity(SphArgs a)
                 d += 0.5f * a.fd_coef * w;
             }
         }
+        if (__builtin_expect(far || strayed, 0)) d = continuity_far<LANES>(a, i, q, nf, nd);
         continuity_finish<LANES, BALLS>(a, a.phf, i, q, d);
     } else {
         const PairSelf s = pair_self<UNIF>(a, i);
@@ -2129,6 +2148,7 @@ struct demsph_sph {
     // lists
     int *nbr_ff = nullptr, *cnt_ff = nullptr, *nbr_fd = nullptr, *cnt_fd = nullptr;
     int* maxcount = nullptr;      // device [2]
+    int* strayed = nullptr;       // device (SphArgs)
     int* maxcount_h = nullptr;    // pinned [2]
     bool lists_valid = false;
     ReadBack read_back;
@@ -2207,7 +2227,7 @@ struct demsph_sph {
         sort_temp = nullptr;
         dfree(cells); dfree(nbr_ff); dfree(cnt_ff); dfree(nbr_fd); dfree(cnt_fd); dfree(DA); dfree(DB); dfree(DC);
         dfree(GR[0]); dfree(GR[1]);
-        dfree(maxcount); dfree(read_back.buf);
+        dfree(maxcount); dfree(strayed); dfree(read_back.buf);
         host_free(maxcount_h);
         maxcount_h = nullptr;
         dfree(DP); dfree(DV); dfree(dphase); dfree(dorig); dfree(dcells); dfree(dummy_near); dfree(d_phases);
@@ -2250,6 +2270,7 @@ struct demsph_sph {
         a.nbr_ff = nbr_ff; a.cnt_ff = cnt_ff; a.nbr_fd = nbr_fd; a.cnt_fd = cnt_fd;
         a.K_ff = K_ff; a.K_fd = K_fd;
         a.fix = fix;
+        a.strayed = strayed;
         const GradK gk = grad_k(phf.hf);
         a.ff_half_invh = (float)(gk.half_invh / fix.inv);
         a.ff_coef = (float)((double)gk.coef * phf.m / fix.inv);
@@ -2388,6 +2409,7 @@ struct demsph_sph {
         GR[0] = dmalloc<GRec>(n); GR[1] = dmalloc<GRec>(n);
         read_back.buf = dmalloc<double>(3 * n);
         maxcount = dmalloc<int>(3);
+        strayed = dmalloc<int>(1);
         DEMSPH_HIP(host_malloc((void**)&maxcount_h, 3 * sizeof(int)));
         alloc_lists();
         cP = cV = cD = cO = 0;
@@ -2508,6 +2530,7 @@ struct demsph_sph {
         ra.odrho = drho[1 - cD];
         ra.cells = cells;
         ra.fix = fix;
+        ra.strayed = strayed;
         ra.oGR = gr(0); ra.rec_full = records_usable() ? 1 : 0;
         DEMSPH_LAUNCH(timer, "sph_reorder", k_reorder, gb, tb, 0, stream, ra);
         cP ^= 1; cV ^= 1; cD ^= 1; cO ^= 1;
@@ -2676,8 +2699,10 @@ struct demsph_sph {
 
     void first_half_enqueue(double dt)
     {
+        if (cG) drop_records();  // a second drift since the search
         SphArgs a = args();
         a.dt = dt;
+        a.stray_vel = (float)(kFixDrift / fix.inv / fabs(dt));
         use_records(a, true);
         if (uniform) momentum_lanes<true, true>("sph_momentum_first", a);
         else momentum_lanes<true, false>("sph_momentum_first", a);
