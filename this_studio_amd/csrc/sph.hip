@@ -585,6 +585,13 @@ __host__ __device__ inline void cut_band(double cut, bool on, float slack, float
     hi = on ? (float)(h * h * (1.0 + 1e-6) + err) : INFINITY;
 }
 
+// What the lanes of a wave wrote to LDS before, its lanes read after.  Costs no
+// instruction: a wave's LDS accesses are in order.
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 __device__ __forceinline__ int rl(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 __device__ __forceinline__ int nth_bit(unsigned m, int n)
 {
@@ -755,8 +762,7 @@ __device__ __forceinline__ void walk_sets(const ListArgs& a, const ListSet& v, i
         // slots lie in the centre row but for some far points
         const int self0 = w0 + kf - runs.o4;
         const bool regular = v.dummy || (self0 >= runs.e3 && self0 + (31 - __clz((int)set)) - kf < runs.e4);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
         int j_next = 0;
         float4 q_next = make_float4(0.f, 0.f, 0.f, 0.f);
         if (total > 0) {
@@ -857,10 +863,10 @@ __device__ __forceinline__ void walk_sets(const ListArgs& a, const ListSet& v, i
                         make_int4(cnt[0] + __popcll(hit[0]), cnt[1] + __popcll(hit[1]), cnt[2] + __popcll(hit[2]),
                                   cnt[3] + __popcll(hit[3]));
             }
+            wave_sync();  // lane 0's counts, for the next candidates
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
         if (lane < G && (set >> lane & 1u)) count = own.count[place];
+        wave_sync();  // read before the next set's are written
     }
     far_pair = fars >> (lane & 31) & 1u;
 }
