@@ -489,6 +489,43 @@ def test_a_particle_that_flies_off_in_one_step(n, cells):
         assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max()
 
 
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_pairs_across_the_ends_of_the_coordinate_range(axis):
+    """A grid of 140 supports on one axis, with the ends of the records' 32-bit
+    range at 64 supports (largest and smallest value side by side) and 128 (zero):
+    lists there against the oracle's, and a step within the tolerances of one
+    step."""
+    rng = np.random.default_rng(axis)
+    dx = 0.01
+    cut = 2.0 * 1.3 * dx
+    side = np.full(3, 4.0 * cut)
+    side[axis] = 140.0 * cut
+    pos = rng.uniform(0.0, 1.0, (1200, 3)) * side
+    g = np.arange(6) * dx
+    block = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3) + rng.uniform(-0.1, 0.1, (216, 3)) * dx
+    pos = [pos]
+    for at in (32.0, 64.0, 96.0, 128.0):
+        c = np.full(3, 0.5 * cut)
+        c[axis] = at * cut - 2.5 * dx
+        pos.append(block + c)
+    pos = np.concatenate(pos)
+    dummy = pos[-216:] + 0.4 * dx
+    spec = scenes.SPHSceneSpec(fluid_pos=pos, dummy_pos=dummy, dx=dx, rho0=1000.0, c0=10.0, nu=1e-6, min_bound=np.zeros(3),
+                               max_bound=side, gravity=np.array([0.0, 0.0, -9.81]), dt=1e-6)
+    o = oracle.OracleSPH(spec)
+    o.neighbor_search()
+    s = make_gpu(spec)
+    s.neighbor_search()
+    assert np.array_equal(s.get("neighborCount"), o.get("count_ff"))
+    assert np.array_equal(s.get("objectPointing"), o.get("pointing_ff"))
+    assert np.array_equal(s.get("dummyObjectPointing"), o.get("pointing_fd"))
+    o = oracle.OracleSPH(spec)
+    s = make_gpu(spec)
+    o.step(spec.dt, 1)
+    s.step(spec.dt, 1)
+    _compare(s, o, 1e-9, 1e-6, 1e-4)
+
+
 @pytest.mark.parametrize("field", ["velocity", "densityChange"])
 def test_records_follow_a_field_set_between_search_and_halves(field, small):
     """A field set after the search reaches the records that the passes

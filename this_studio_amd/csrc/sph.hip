@@ -124,8 +124,12 @@ struct Fix3 {
 __device__ __forceinline__ int fix_coord(double X)
 {
     const double y = X + 0.5;
-    return (int)(unsigned)(y - 4294967296.0 * floor(y * (1.0 / 4294967296.0)));
+    // fmin: the remainder can round up to 2^32, and no number converts
+    return (int)(unsigned)fmin(y - 4294967296.0 * floor(y * (1.0 / 4294967296.0)), 4294967295.0);
 }
+// The difference of two coordinates, modulo 2^32: both ends of the range of int
+// meet wherever a grid is longer than 32 edges.
+__device__ __forceinline__ float fix_diff(int a, int b) { return (float)(int)((unsigned)a - (unsigned)b); }
 __device__ __forceinline__ bool fix_out(double X, double E) { return !(X >= -kFixPad && X <= E + kFixPad); }
 __device__ __forceinline__ bool fix_edge(double X, double E)
 {
@@ -716,7 +720,7 @@ __device__ __forceinline__ void walk_sets(const ListArgs& a, const ListSet& v, i
             own.count[ns + lane] = own.base[ns + lane] = own.self[ns + lane] = 0;
         }
         if (lane < G && (set >> lane & 1u)) {
-            const float x = (float)(qx - rx), y = (float)(qy - ry), z = (float)(qz - rz);
+            const float x = fix_diff(qx, rx), y = fix_diff(qy, ry), z = fix_diff(qz, rz);
             const float n2 = x * x + y * y + z * z;
             float lo = v.lo, hi = v.hi, w = n2;
             if (!UNIF) cut_band(2.0 * h * a.inv, a.prefilter != 0, kListSlack, a.err, lo, hi);
@@ -777,8 +781,8 @@ __device__ __forceinline__ void walk_sets(const ListArgs& a, const ListSet& v, i
                 q_next = v.A[j_next];
             }
             const bool in = t0 + lane < total;
-            const float x = (float)(__float_as_int(q.x) - rx), y = (float)(__float_as_int(q.y) - ry),
-                        z = (float)(__float_as_int(q.z) - rz);
+            const float x = fix_diff(__float_as_int(q.x), rx), y = fix_diff(__float_as_int(q.y), ry),
+                        z = fix_diff(__float_as_int(q.z), rz);
             const float n2 = in ? (q.w == -2.0f ? kFixMiss : x * x + y * y + z * z) : INFINITY;
             const unsigned long long inm = __ballot(in), farm = __ballot(q.w < 0.0f) & inm;
             const unsigned long long cold = regular ? (inner ? __ballot(q.w == -1.0f) & inm : farm) : inm;
@@ -901,9 +905,9 @@ __global__ __launch_bounds__(kThreads, 6) void k_build_lists(ListArgs a, int per
         const int nxy = g.nx * g.ny;
         const int cz = cell / nxy, cy = (cell - cz * nxy) / g.nx, cx = cell - cz * nxy - cy * g.nx;
         const double h = UNIF ? a.hf : a.phases[phase_bits(a.V[i].w)].h;
-        const float x = (float)(__float_as_int(r.x) - cell_middle(cx, a.stepx)),
-                    y = (float)(__float_as_int(r.y) - cell_middle(cy, a.stepy)),
-                    z = (float)(__float_as_int(r.z) - cell_middle(cz, a.stepz));
+        const float x = fix_diff(__float_as_int(r.x), cell_middle(cx, a.stepx)),
+                    y = fix_diff(__float_as_int(r.y), cell_middle(cy, a.stepy)),
+                    z = fix_diff(__float_as_int(r.z), cell_middle(cz, a.stepz));
         const bool plain = !far && fmaxf(fmaxf(fabsf(x), fabsf(y)), fabsf(z)) < a.reach;
         const unsigned live = n == 32 ? ~0u : (1u << n) - 1u;
         unsigned dnear = 0;
@@ -1115,7 +1119,7 @@ struct PairDist {
 __device__ __forceinline__ PairDist pair_dist(int ax, int ay, int az, int bx, int by, int bz, float half_invh_u)
 {
     PairDist d;
-    d.x = (float)(ax - bx); d.y = (float)(ay - by); d.z = (float)(az - bz);
+    d.x = fix_diff(ax, bx); d.y = fix_diff(ay, by); d.z = fix_diff(az, bz);
     const float r2 = d.x * d.x + d.y * d.y + d.z * d.z;
     // distances are whole units: only zero is below 1
     d.inv_r = rsq(fmaxf(r2, 0.25f));
@@ -1784,8 +1788,8 @@ __global__ __launch_bounds__(256) void k_fs_rev_walk(RevArgs a)
             if (UNIF) {
                 if (i < e) {
                     const float4 q = a.A[i];
-                    const float fx = (float)(__float_as_int(q.x) - bq.x), fy = (float)(__float_as_int(q.y) - bq.y),
-                                fz = (float)(__float_as_int(q.z) - bq.z);
+                    const float fx = fix_diff(__float_as_int(q.x), bq.x), fy = fix_diff(__float_as_int(q.y), bq.y),
+                                fz = fix_diff(__float_as_int(q.z), bq.z);
                     const float d2 = fx * fx + fy * fy + fz * fz;
                     hit = d2 < lo;
                     if (!(q.w > 0.f) || (d2 < hi && !hit)) {
