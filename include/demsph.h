@@ -199,10 +199,10 @@ int demsph_sph_graph_captures(demsph_sph* s, long* count);
  * fixed-point positions and only those within rounding of the cut (or far
  * outside the grid) in exact FP64, 0 tests all in FP64; both give
  * the same lists.  "pairRecords": 1 (default) lets the pair passes of a
- * one-phase scene gather 32-byte records holding each neighbour's position
- * in fixed point (32 bits an axis, 2^25 units or more to the largest cell
- * edge), 0 gathers the FP64 positions;
- * results differ by FP32 rounding.  demsph_sph_tune_get reads the value in
+ * one-phase scene gather 32-byte records holding each fluid neighbour's
+ * position in fixed point (32 bits an axis, 2^25 units or more to the largest
+ * cell edge; dummies keep FP64 positions), 0 gathers FP64 positions; results
+ * differ by FP32 rounding.  demsph_sph_tune_get reads the value in
  * effect ("pairRecords": 1 only where the records are in use). */
 int demsph_sph_tune(demsph_sph* s, const char* knob, int value);
 int demsph_sph_tune_get(demsph_sph* s, const char* knob, int* value);

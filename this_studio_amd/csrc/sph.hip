@@ -114,7 +114,6 @@ struct FixGeom {
     double minx, miny, minz;
     double ex, ey, ez;  // extent of the grid in units
     double inv;         // units per metre
-    float u;            // metres per unit
     double edge;        // the edge, in units
 };
 struct Fix3 {
@@ -199,6 +198,18 @@ __host__ __device__ constexpr int list_count(int c) { return c & (kFarBit - 1); 
 
 __device__ __forceinline__ unsigned phase_bits(float w) { return __float_as_uint(w); }
 
+// A constant in two floats.  Rounded to one it is off by the same up to 6e-8 of
+// itself in every pair or particle, which no sum averages out.
+struct Split {
+    float hi, lo;
+};
+inline Split split(double v)
+{
+    const float hi = (float)v;
+    return Split{hi, (float)(v - (double)hi)};
+}
+__device__ __forceinline__ float times(float v, const Split& k) { return fmaf(v, k.lo, v * k.hi); }
+
 struct SphArgs {
     int nf, nd;
     const Phase* phases;
@@ -222,14 +233,13 @@ struct SphArgs {
     FixGeom fix;
     int* strayed;    // set by the first half's pass when a point moves farther than records allow
     float stray_vel;  // velocity above which it does (sum over the axes)
-    // fluid and dummy pairs on records: u / 2h, u m_j times the kernel constant (GradK)
-    float ff_half_invh, ff_coef, fd_half_invh, fd_coef;
+    // pairs in units of the records: u / 2h (of fluid pairs a power of two) and
+    // u m_j times the kernel constant (GradK)
+    float ff_half_invh;
+    Split ff_coef, fd_half_invh, fd_coef;
     // dummies (sorted once)
     const DummyPos* DP;
     const float4* DV;
-    // their records: {qx, qy, qz, -}, {nx, ny, nz, vx}, {vy, vz}
-    const float4 *DA, *DB;
-    const float2* DC;
     const uint8_t* dphase;
     // coupled DEM balls (solids), sorted into the fluid grid each step
     int ns;
@@ -240,6 +250,7 @@ struct SphArgs {
     float* acs;             // per fluid slot: coupling acceleration of the last pass (3 floats), or null
     // physics
     float gx, gy, gz;
+    Split gu[3];  // gravity times u
     double dt;
     int eos;
     float gamma, inv_gamma;
@@ -1036,10 +1047,6 @@ struct DummyRec {
     DummyPos D;
     float4 V;
 };
-struct DummyFix {
-    float4 A, B;
-    float2 C;
-};
 
 // Sum over the LANES lanes of a particle (a fixed butterfly order).
 template <int LANES, class T>
@@ -1162,42 +1169,56 @@ __device__ __forceinline__ void continuity_ff_g(const PairSelf& s, const GRec& R
     sum += d.t3 * rcp(R.rho * rc) * num;
 }
 
-// momentum_fd and continuity_fd on records; a lane's entries past the end
-// count as out of reach.
-__device__ __forceinline__ PairDist dummy_dist(const SphArgs& a, const PairSelf& s, const DummyFix& R, bool valid,
+// momentum_fd and continuity_fd with the factors of a pass taken out; a lane's
+// entries past the end count as out of reach.  Dummy pairs are few (2 of 78 of a
+// particle in the 256k dam break) and keep FP64 positions, differenced before
+// they are rounded; on records the steps took the same time.  Distances are in
+// the records' units all the same: the hardware's 1/sqrt is off by up to an ulp
+// in a way that depends on the mantissa, the same for many pairs of a lattice,
+// and fluid and dummy terms oppose each other at a wall.  In metres their errors
+// did not cancel (velocities after 50 steps of 40k particles off by 7.4e-8, now
+// 4.6e-8).  An error of 1/2h counts three times over in (1 - r/2h)^3, and more
+// near the cut: hence two floats.
+__device__ __forceinline__ PairDist dummy_dist(const SphArgs& a, const PairSelf& s, const DummyRec& R, bool valid,
                                                float& PR, float& rhoj)
 {
-    PairDist d = pair_dist(s.qx, s.qy, s.qz, __float_as_int(R.A.x), __float_as_int(R.A.y), __float_as_int(R.A.z),
-                           a.fd_half_invh);
-    d.t3 = valid ? d.t3 : 0.0f;
-    const float grj = fmaxf(-(a.gx * d.x + a.gy * d.y + a.gz * d.z) * a.fix.u, 0.0f);
+    PairDist d;
+    d.x = (float)((s.x - R.D.x) * a.fix.inv);
+    d.y = (float)((s.y - R.D.y) * a.fix.inv);
+    d.z = (float)((s.z - R.D.z) * a.fix.inv);
+    const float r2 = d.x * d.x + d.y * d.y + d.z * d.z;
+    d.inv_r = rsq(fmaxf(r2, 1e-6f));
+    d.r = r2 * d.inv_r;
+    const float t = fmaxf(fmaf(-d.r, a.fd_half_invh.lo, fmaf(-d.r, a.fd_half_invh.hi, 1.0f)), 0.0f);
+    d.t3 = valid ? t * t * t : 0.0f;
+    const float grj = fmaxf(-(times(d.x, a.gu[0]) + times(d.y, a.gu[1]) + times(d.z, a.gu[2])), 0.0f);
     PR = s.p + s.rho * grj;
     rhoj = dummy_rho(a, a.phd, PR);
     return d;
 }
-__device__ __forceinline__ void momentum_fd_g(const SphArgs& a, const PairSelf& s, const DummyFix& R, bool valid,
+__device__ __forceinline__ void momentum_fd_g(const SphArgs& a, const PairSelf& s, const DummyRec& R, bool valid,
                                               MomentumSums& m)
 {
     float PR, rhoj;
     const PairDist d = dummy_dist(a, s, R, valid, PR, rhoj);
-    const float nx = R.B.x, ny = R.B.y, nz = R.B.z;
+    const float nx = R.D.nx, ny = R.D.ny, nz = R.V.w;
     const float UL = -(nx * s.vx + ny * s.vy + nz * s.vz);
-    const float UR = -UL - 2.0f * (nx * R.B.w + ny * R.C.x + nz * R.C.y);
+    const float UR = -UL - 2.0f * (nx * R.V.x + ny * R.V.y + nz * R.V.z);
     const float cbar = 0.5f * (s.ph.c + a.phd.c), rbar = 0.5f * (s.rho + rhoj);
     const float beta = fminf(3.0f * fmaxf(UL - UR, 0.0f), cbar);
     const float Ps2 = (s.p + PR) + beta * rbar * (UL - UR);
     const float w = d.t3 * rcp(rhoj);
     const float kp = Ps2 * w, kv = d.r * w;
     m.px += kp * d.x; m.py += kp * d.y; m.pz += kp * d.z;
-    m.vx += kv * (s.vx - R.B.w); m.vy += kv * (s.vy - R.C.x); m.vz += kv * (s.vz - R.C.y);
+    m.vx += kv * (s.vx - R.V.x); m.vy += kv * (s.vy - R.V.y); m.vz += kv * (s.vz - R.V.z);
 }
-__device__ __forceinline__ void continuity_fd_g(const SphArgs& a, const PairSelf& s, const DummyFix& R, bool valid,
+__device__ __forceinline__ void continuity_fd_g(const SphArgs& a, const PairSelf& s, const DummyRec& R, bool valid,
                                                 float& sum)
 {
     float PR, rhoj;
     const PairDist d = dummy_dist(a, s, R, valid, PR, rhoj);
     const float cbar = 0.5f * (s.ph.c + a.phd.c), rbar = 0.5f * (s.rho + rhoj);
-    const float t = (s.vx - R.B.w) * d.x + (s.vy - R.C.x) * d.y + (s.vz - R.C.y) * d.z +
+    const float t = (s.vx - R.V.x) * d.x + (s.vy - R.V.y) * d.y + (s.vz - R.V.z) * d.z +
                     (s.p - PR) * d.r * rcp(rbar * cbar);
     sum += d.t3 * rcp(rhoj) * t;
 }
@@ -1485,24 +1506,25 @@ __global__ __launch_bounds__(kThreads) void k_momentum(SphArgs a)
         if (!far) {
             int pre[kPreEntries];
             preload_entries<LANES>(a.nbr_ff, a.K_ff, i, q, pre);
-            const PairSelf s = pair_self_rec(a, i);
+            PairSelf s = pair_self_rec(a, i);
             const float half_invh_u = a.ff_half_invh, half_c = 0.5f * s.ph.c;
             MomentumSums m{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
             for_entries_pre<LANES>(pre, a.nbr_ff, nf, a.K_ff, i, q, i, [&](int j) { return ld_grec(a.GRin, a.nf, j); },
                                    [&](const GRec& R, int, bool) { momentum_ff_g(s, R, half_invh_u, half_c, m); });
-            const float k = a.ff_coef * s.inv_rho, kv = 2.0f * s.ph.nu * k;
-            ax = kv * m.vx - k * m.px;
-            ay = kv * m.vy - k * m.py;
-            az = kv * m.vz - k * m.pz;
+            const float nu2 = 2.0f * s.ph.nu;
+            ax = times((nu2 * m.vx - m.px) * s.inv_rho, a.ff_coef);
+            ay = times((nu2 * m.vy - m.py) * s.inv_rho, a.ff_coef);
+            az = times((nu2 * m.vz - m.pz) * s.inv_rho, a.ff_coef);
             if (nd > 0) {
+                s.x = a.P[i].x; s.y = a.P[i].y; s.z = a.P[i].z;
                 MomentumSums w{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
                 for_entries<LANES>(a.nbr_fd, nd, a.K_fd, i, q, 0,
-                                   [&](int j) { return DummyFix{ld_at(a.DA, j), ld_at(a.DB, j), ld_at(a.DC, j)}; },
-                                   [&](const DummyFix& R, int, bool valid) { momentum_fd_g(a, s, R, valid, w); });
-                const float kd = a.fd_coef * s.inv_rho, kvd = (s.ph.nu + a.phd.nu) * kd;
-                ax += kvd * w.vx - kd * w.px;
-                ay += kvd * w.vy - kd * w.py;
-                az += kvd * w.vz - kd * w.pz;
+                                   load_d,
+                                   [&](const DummyRec& R, int, bool valid) { momentum_fd_g(a, s, R, valid, w); });
+                const float nu = s.ph.nu + a.phd.nu;
+                ax += times((nu * w.vx - w.px) * s.inv_rho, a.fd_coef);
+                ay += times((nu * w.vy - w.py) * s.inv_rho, a.fd_coef);
+                az += times((nu * w.vz - w.pz) * s.inv_rho, a.fd_coef);
             }
         }
         if (__builtin_expect(far || strayed, 0)) {
@@ -1638,17 +1660,18 @@ __global__ __launch_bounds__(kThreads) void k_continuity(SphArgs a)
         if (!far) {
             int pre[kPreEntries];
             preload_entries<LANES>(a.nbr_ff, a.K_ff, i, q, pre);
-            const PairSelf s = pair_self_rec(a, i);
+            PairSelf s = pair_self_rec(a, i);
             const float half_invh_u = a.ff_half_invh, half_c = 0.5f * s.ph.c, rho_c = s.rho * half_c;
             for_entries_pre<LANES>(pre, a.nbr_ff, nf, a.K_ff, i, q, i, [&](int j) { return ld_grec(a.GRin, a.nf, j); },
                                    [&](const GRec& R, int, bool) { continuity_ff_g(s, R, half_invh_u, half_c, rho_c, d); });
-            d *= 0.5f * a.ff_coef;
+            d = times(0.5f * d, a.ff_coef);
             if (nd > 0) {
+                s.x = a.P[i].x; s.y = a.P[i].y; s.z = a.P[i].z;
                 float w = 0.f;
                 for_entries<LANES>(a.nbr_fd, nd, a.K_fd, i, q, 0,
-                                   [&](int j) { return DummyFix{ld_at(a.DA, j), ld_at(a.DB, j), ld_at(a.DC, j)}; },
-                                   [&](const DummyFix& R, int, bool valid) { continuity_fd_g(a, s, R, valid, w); });
-                d += 0.5f * a.fd_coef * w;
+                                   load_d,
+                                   [&](const DummyRec& R, int, bool valid) { continuity_fd_g(a, s, R, valid, w); });
+                d += times(0.5f * w, a.fd_coef);
             }
         }
         if (__builtin_expect(far || strayed, 0)) d = continuity_far<LANES>(a, i, q, nf, nd);
@@ -2024,19 +2047,6 @@ __global__ void k_dummy_near(GridGeom g, long long numGrids, const int2* __restr
     near[c] = any;
 }
 
-// The rest of the dummies' records, once their normals are known.
-__global__ __launch_bounds__(kThreads) void k_dummy_records(int n, const DummyPos* __restrict__ DP,
-                                                            const float4* __restrict__ DV, float4* __restrict__ DB,
-                                                            float2* __restrict__ DC)
-{
-    const int k = blockIdx.x * kThreads + threadIdx.x;
-    if (k >= n) return;
-    const DummyPos d = DP[k];
-    const float4 v = DV[k];
-    DB[k] = make_float4(d.nx, d.ny, v.w, v.x);
-    DC[k] = make_float2(v.y, v.z);
-}
-
 __global__ void k_dummy_hash(int n, GridGeom g, const double* __restrict__ px, const double* __restrict__ py,
                              const double* __restrict__ pz, uint32_t* __restrict__ key)
 {
@@ -2140,6 +2150,8 @@ struct demsph_sph {
     bool fluid_uniform() const { return fluid_one_phase; }
     SolidView solids;      // coupled balls (ns == 0 outside coupled stepping)
     Phase phf{}, phd{};
+    std::vector<double> phase_m;        // masses of the phases
+    double mass_f = 0.0, mass_d = 0.0;  // of phf and phd
 
     // fluid state, double-buffered per record group
     FluidPos* P[2] = {};
@@ -2211,8 +2223,7 @@ struct demsph_sph {
     int pair_lanes_set = 0;  // 0: chosen from the particle count
     int list_lanes_set = 0;
     bool prefilter = true;  // list candidates outside the cut's band are decided in fixed point
-    float4 *DA = nullptr, *DB = nullptr;  // dummy records (SphArgs)
-    float2* DC = nullptr;
+    float4* DA = nullptr;    // the dummies' fixed-point positions
 
     std::vector<demsph_couple*> couples;  // couplings holding this scene
 
@@ -2235,7 +2246,7 @@ struct demsph_sph {
         dfree(rank); dfree(key); dfree(skey); dfree(ktmp); dfree(perm); dfree(vtmp);
         dev_free(sort_temp);
         sort_temp = nullptr;
-        dfree(cells); dfree(nbr_ff); dfree(cnt_ff); dfree(nbr_fd); dfree(cnt_fd); dfree(DA); dfree(DB); dfree(DC);
+        dfree(cells); dfree(nbr_ff); dfree(cnt_ff); dfree(nbr_fd); dfree(cnt_fd); dfree(DA);
         dfree(GR[0]); dfree(GR[1]);
         dfree(maxcount); dfree(strayed); dfree(read_back.buf);
         host_free(maxcount_h);
@@ -2267,6 +2278,7 @@ struct demsph_sph {
         q.c2 = (float)(c * c);
         q.taitB = (float)(r0 * c * c / gamma);
         phases.push_back(q);
+        phase_m.push_back(m);
         return (uint8_t)(phases.size() - 1);
     }
 
@@ -2281,16 +2293,17 @@ struct demsph_sph {
         a.K_ff = K_ff; a.K_fd = K_fd;
         a.fix = fix;
         a.strayed = strayed;
-        const GradK gk = grad_k(phf.hf);
-        a.ff_half_invh = (float)(gk.half_invh / fix.inv);
-        a.ff_coef = (float)((double)gk.coef * phf.m / fix.inv);
-        const GradK gd = grad_k(0.5f * (phf.hf + phd.hf));
-        a.fd_half_invh = (float)(gd.half_invh / fix.inv);
-        a.fd_coef = (float)((double)gd.coef * phd.m / fix.inv);
-        a.DP = DP; a.DV = DV; a.dphase = dphase; a.DA = DA; a.DB = DB; a.DC = DC;
+        const auto coef = [](double h) { return -105.0 / (16.0 * M_PI) / (h * h * h * h * h); };
+        const double hd = 0.5 * (phf.h + phd.h);
+        a.ff_half_invh = (float)(0.5 / (phf.h * fix.inv));
+        a.ff_coef = split(coef(phf.h) * mass_f / fix.inv);
+        a.fd_half_invh = split(0.5 / (hd * fix.inv));
+        a.fd_coef = split(coef(hd) * mass_d / fix.inv);
+        a.DP = DP; a.DV = DV; a.dphase = dphase;
         a.ns = solids.ns; a.SP = solids.SP; a.SV = solids.SV; a.SW = solids.SW;
         a.nbr_fs = solids.nbr_fs; a.cnt_fs = solids.cnt_fs; a.K_fs = solids.K_fs; a.acs = solids.acs;
         a.gx = (float)g[0]; a.gy = (float)g[1]; a.gz = (float)g[2];
+        for (int k = 0; k < 3; k++) a.gu[k] = split(g[k] / fix.inv);
         a.eos = eos;
         a.gamma = (float)gamma;
         a.inv_gamma = (float)(1.0 / gamma);
@@ -2342,7 +2355,7 @@ struct demsph_sph {
                                  + 3 * sizeof(double)                     // read-back
                                  + sizeof(int) * (size_t)(round_chunk(K_ff) + round_chunk(K_fd));
         const size_t per_sort = 3 * sizeof(uint32_t) + 2 * sizeof(int);
-        const size_t per_dummy = sizeof(DummyPos) + 3 * sizeof(float4) + sizeof(float2) + 1 + sizeof(int);
+        const size_t per_dummy = sizeof(DummyPos) + 2 * sizeof(float4) + 1 + sizeof(int);
         // initialisation uploads positions, velocities and phases through
         // temporary buffers, which the runtime's allocator keeps cached
         const size_t upload = 6 * sizeof(double) + 1;
@@ -2368,6 +2381,7 @@ struct demsph_sph {
         if (numGrids > INT32_MAX / 2) throw InvalidArg("grid too large");
 
         phases.clear();
+        phase_m.clear();
         fphase_h.resize(nf);
         dphase_h.resize(nd);
         for (int i = 0; i < nf; i++) {
@@ -2385,6 +2399,8 @@ struct demsph_sph {
         fluid_one_phase = fu;
         phf = phases[fphase_h[0]];
         phd = nd > 0 ? phases[dphase_h[0]] : phf;
+        mass_f = phase_m[fphase_h[0]];
+        mass_d = nd > 0 ? phase_m[dphase_h[0]] : mass_f;
         d_phases = dmalloc<Phase>(phases.size());
         DEMSPH_HIP(hipMemcpyAsync(d_phases, phases.data(), sizeof(Phase) * phases.size(), hipMemcpyHostToDevice, stream));
 
@@ -2401,16 +2417,16 @@ struct demsph_sph {
         DEMSPH_HIP(dev_malloc(&sort_temp, radix_sort_temp_bytes(nsort)));
         cells = dmalloc<int2>(numGrids);
         const size_t md = nd > 0 ? nd : 1;
-        DA = dmalloc<float4>(md); DB = dmalloc<float4>(md); DC = dmalloc<float2>(md);
+        DA = dmalloc<float4>(md);
         {
             fix.minx = grid.minx; fix.miny = grid.miny; fix.minz = grid.minz;
-            // a power of two of units to the fluid's 2 h makes the kernel
-            // argument r / 2h exact in the pair passes
+            // a power of two of units to the fluid's 2 h: u / 2h is exact in
+            // the pair passes.  Its rounding is the same for every pair and
+            // counts three times over in (1 - r/2h)^3 near the cut.
             const double emax = std::max(std::max(grid.cx, cell), std::max(grid.cy, grid.cz)),
-                         two_h = 1.0 / grad_k(phf.hf).half_invh;
-            fix.inv = two_h <= emax && emax <= 2.0 * two_h ? 0.5 * kFixPerEdge / two_h : kFixPerEdge / emax;
+                         two_h = 2.0 * phf.h;
+            fix.inv = std::ldexp(kFixPerEdge / two_h, -(int)std::ceil(std::log2(emax / two_h) - 1e-9));
             fix.edge = emax * fix.inv;
-            fix.u = (float)(1.0 / fix.inv);
             fix.ex = (grid.maxx - grid.minx) * fix.inv;
             fix.ey = (grid.maxy - grid.miny) * fix.inv;
             fix.ez = (grid.maxz - grid.minz) * fix.inv;
@@ -2482,8 +2498,6 @@ struct demsph_sph {
             na.nd = (int)m; na.grid = grid; na.phases = d_phases; na.DP = DP; na.DV = DV;
             na.dphase = dphase; na.dcells = dcells;
             hipLaunchKernelGGL(k_dummy_normals, dim3(blocks_for(m, kThreads)), dim3(kThreads), 0, stream, na);
-            hipLaunchKernelGGL(k_dummy_records, dim3(blocks_for(m, kThreads)), dim3(kThreads), 0, stream, (int)m, DP,
-                               DV, DB, DC);
             DEMSPH_HIP(hipGetLastError());
             DEMSPH_HIP(hipStreamSynchronize(stream));
             dfree(ux); dfree(uy); dfree(uz); dfree(wx); dfree(wy); dfree(wz); dfree(uph);
