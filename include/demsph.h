@@ -212,8 +212,8 @@ int demsph_sph_tune_get(demsph_sph* s, const char* knob, int* value);
  * untimed step and then trialSteps timed steps (HIP events) from a
  * checkpoint that is restored afterwards, so the scene's state and its
  * later results are those of a scene never tuned with the chosen knobs.
- * mode 0 tries only result-invariant knobs (listLanes 1, 2, 4, 8 with and
- * without listPrefilter: every variant builds the same lists); mode 1 also
+ * mode 0 tries only result-invariant knobs (listLanes 2, 4, 8 with and without
+ * listPrefilter, 1 with it: every variant builds the same lists); mode 1 also
  * tries pairLanes (FP32 summation order changes).  A variant within 2 % of
  * the built-in rule keeps the rule.  The cell size is not tuned: it fixes
  * the list order and the sort (2 max h, WCSPHSolver.h:127-135).  The choice

@@ -3043,12 +3043,13 @@ struct demsph_sph {
         };
         TuneChoice best;
         try {
-            // List build: every lane count, with and without the prefilter
-            // (one lane has no prefilter variant).  Near-ties keep the rule.
+            // List build: every lane count, with and without the prefilter;
+            // one lane (64 particles a wave) with it only.  Near-ties keep the
+            // rule.
             double best_l = 0.0, pair_sum = 0.0;
             for (int L : {1, 2, 4, 8}) {
                 for (int pre = 0; pre < 2; pre++) {
-                    if (L == 1 && pre) continue;
+                    if (L == 1 && !pre) continue;
                     list_lanes_set = L;
                     prefilter = pre != 0;
                     const auto t = time_trial(dt, steps, sP, sV, sD, sO);
