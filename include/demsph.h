@@ -136,7 +136,9 @@ int demsph_sph_sizes(demsph_sph* s, size_t* numFluid, size_t* numDummy, size_t* 
  * (int, numGrids)  "neighborCount" "dummyNeighborCount" (int, n)
  * "objectPointing" "dummyObjectPointing" (int, total pairs: the reference's
  * pair list, grouped by pointed particle in insertion order).
- * *count receives the element count; out may be NULL to query it. */
+ * *count receives the element count; out may be NULL to query it.
+ * Several threads may read one scene at a time (not beside calls that change
+ * it). */
 int demsph_sph_get(demsph_sph* s, const char* field, void* out, size_t capacity, size_t* count);
 
 /* Frame files: the reference's outputWCSPHVTU (WCSPHSolver.h:360-443,
@@ -377,7 +379,8 @@ int demsph_dem_sizes(demsph_dem* d, size_t* numBalls, size_t* numClumps, size_t*
  * "clumpPosition" "clumpVelocity" "clumpAngularVelocity" (double 3/clump),
  * "clumpOrientation" (double 4/clump), "wallPosition" (double 3/wall),
  * "wallOrientation" (double 4/wall), "vertexGlobalPosition" (double 3/vertex),
- * "hashValue" "hashIndex" "cellHashStart" "cellHashEnd" (int). */
+ * "hashValue" "hashIndex" "cellHashStart" "cellHashEnd" (int).
+ * Several threads may read one scene at a time, as with demsph_sph_get. */
 int demsph_dem_get(demsph_dem* d, const char* field, void* out, size_t capacity, size_t* count);
 
 /* Frame files: the reference's outputBallVTU (DEMSolver.h:908-993,

@@ -184,11 +184,10 @@ def test_lane_settings_build_identical_lists_and_agree(small):
 
 
 def test_gather_records_agree_with_fp64_records():
-    """The pair passes gather 32-byte records holding each neighbour's
-    position as an FP32 offset from its cell's origin, its cell relative to
-    the particle's stencil centre coded in the list entry (pairRecords 1), or
-    the FP64 positions themselves (pairRecords 0).  The lists export the
-    same; the steps agree to FP32 rounding, and both stay deterministic."""
+    """The pair passes gather 32-byte records holding each fluid neighbour's
+    position in 32-bit fixed point (pairRecords 1), or the FP64 positions
+    themselves (pairRecords 0).  The lists are the same; the steps agree to
+    FP32 rounding, and both stay deterministic."""
     spec = scenes.dam_break(dx=0.01)  # 40 x 40 x 20 fluid
     runs, lists = {}, {}
     for mode in (1, 0, 1):
@@ -212,8 +211,8 @@ def test_gather_records_agree_with_fp64_records():
 def test_gather_records_outside_the_grid_match_oracle():
     """With the grid's top face below the column's top row and the tank's
     upper dummies, those particles hash into the top layer of cells
-    (clamped) while lying outside it: their gather records hold offsets of
-    more than a cell, and a stencil centre can differ from the hashed cell.
+    (clamped) while lying outside it, and a stencil centre can differ from the
+    hashed cell.
     Both record forms still match the FP64 oracle over 50 steps."""
     spec = scenes.small_dam_break()
     spec.max_bound = np.array(spec.max_bound, dtype=float)

@@ -19,14 +19,16 @@
 // Neighbour lists hold K entries per slot in 32-byte chunks of eight, those
 // of 16 consecutive slots interleaved (list_entry): the lanes of a wavefront
 // read one chunk of consecutive slots as consecutive 16-byte words, and the
-// list build finds an entry with one multiply-add.  Each slot's list holds neighbour slots in the reference's
-// exact walk order (z, y, x cells, then ascending insertion index), so the
-// pair set and its per-particle order are identical to the reference's.  The
+// list build finds an entry with one multiply-add.  Each slot's list holds
+// neighbour slots in the reference's exact walk order (z, y, x cells, then
+// ascending insertion index), so the pair set and its per-particle order are
+// identical to the reference's.  The
 // lists of coupled balls are ELL in 32-byte chunks: entries 8c..8c+7 of slot
 // i at int offset (c*n + i)*8.
 //
-// Pair arithmetic is FP32 (positions differenced in FP64 first); state
-// integration is FP64.
+// Pair arithmetic is FP32.  Positions are differenced before they are rounded
+// to it: fluid neighbours of uniform scenes as 32-bit fixed point (FixGeom),
+// all other pairs in FP64.  State integration is FP64.
 #include "common.hpp"
 #include "internal.hpp"
 #include "timing.hpp"
@@ -2585,8 +2587,10 @@ struct demsph_sph {
     // particles): the fewest of 2, 4, 8 that put 600k threads in flight.
     // More particles a wave share more of its candidate loads, and fewer
     // waves hide less of each other's latencies.  Measured with 8 / 4 / 2
-    // lanes, us: 2k particles 26 / 36 / 55, 18k 31 / 39 / 63, 60k 54 / 56 /
-    // 80, 256k 137 / 125 / 134, 1M 443 / 355 / 330.
+    // lanes, us: 2k particles 18 / 27 / 42, 18k 25 / 32 / 51, 60k 49 / 47 / 53,
+    // 256k 131 / 117 / 134 (a dam break on its lattice 135 / 134 / 183), 1M 432 /
+    // 341 / 320.  Lanes that each walked their own particle's candidates took
+    // 24, 30, 51, 126 (129) and 428.
     int list_lanes() const
     {
         if (list_lanes_set > 0) return list_lanes_set;
