@@ -562,6 +562,38 @@ def test_records_lose_nothing_beside_dummies(ratio):
         assert a <= max(2.0 * b, 2e-7)
 
 
+@pytest.mark.parametrize("first_only", [False, True])
+def test_fluid_without_support(first_only):
+    """Fluid particles of spacing zero (all of them, or the first one) over
+    dummies: they have no support of their own, lists equal the oracle's and a
+    step gives what the FP64 records give (1e-5 of the largest value, as for
+    FP32 sums in another order) and no infinities."""
+    rng = np.random.default_rng(2)
+    dx = 0.01
+    pos = rng.uniform(0.0, 0.1, (300, 3)) * [1.0, 1.0, 0.3]
+    g = np.arange(0.0, 0.1, dx)
+    dummy = np.stack(np.meshgrid(g, g, [-0.5 * dx], indexing="ij"), -1).reshape(-1, 3)
+    spec = scenes.SPHSceneSpec(fluid_pos=pos, dummy_pos=dummy, dx=dx, rho0=1000.0, c0=10.0, nu=1e-6,
+                               min_bound=np.array([0.0, 0.0, -dx]), max_bound=np.full(3, 0.1),
+                               gravity=np.array([0.0, 0.0, -9.81]), dt=1e-6)
+    spec.fluid_dx = np.zeros(300) if not first_only else np.where(np.arange(300) == 0, 0.0, dx)
+    o = oracle.OracleSPH(spec)
+    o.neighbor_search()
+    got = []
+    for rec in (1, 0):
+        s = make_gpu(spec)
+        s.tune("pairRecords", rec)
+        s.neighbor_search()
+        assert np.array_equal(s.get("neighborCount"), o.get("count_ff"))
+        assert np.array_equal(s.get("objectPointing"), o.get("pointing_ff"))
+        assert np.array_equal(s.get("dummyObjectPointing"), o.get("pointing_fd"))
+        s.step(spec.dt, 1)
+        got.append([s.get(f) for f in ("position", "velocity", "density")])
+    for a, b in zip(*got):
+        assert np.isfinite(a).all()
+        assert np.abs(a - b).max() <= 1e-5 * np.abs(b).max()
+
+
 @pytest.mark.parametrize("field", ["velocity", "densityChange"])
 def test_records_follow_a_field_set_between_search_and_halves(field, small):
     """A field set after the search reaches the records that the passes

@@ -2295,7 +2295,8 @@ struct demsph_sph {
         a.K_ff = K_ff; a.K_fd = K_fd;
         a.fix = fix;
         a.strayed = strayed;
-        const auto coef = [](double h) { return -105.0 / (16.0 * M_PI) / (h * h * h * h * h); };
+        // no support, no pairs: not an infinite constant times an empty sum
+        const auto coef = [](double h) { return h > 0.0 ? -105.0 / (16.0 * M_PI) / (h * h * h * h * h) : 0.0; };
         const double hd = 0.5 * (phf.h + phd.h);
         a.ff_half_invh = (float)(0.5 / (phf.h * fix.inv));
         a.ff_coef = split(coef(phf.h) * mass_f / fix.inv);
@@ -2427,7 +2428,8 @@ struct demsph_sph {
             // counts three times over in (1 - r/2h)^3 near the cut.
             const double emax = std::max(std::max(grid.cx, cell), std::max(grid.cy, grid.cz)),
                          two_h = 2.0 * phf.h;
-            fix.inv = std::ldexp(kFixPerEdge / two_h, -(int)std::ceil(std::log2(emax / two_h) - 1e-9));
+            fix.inv = two_h > 0.0 ? std::ldexp(kFixPerEdge / two_h, -(int)std::ceil(std::log2(emax / two_h) - 1e-9))
+                                  : kFixPerEdge / emax;
             fix.edge = emax * fix.inv;
             fix.ex = (grid.maxx - grid.minx) * fix.inv;
             fix.ey = (grid.maxy - grid.miny) * fix.inv;
